@@ -138,60 +138,56 @@ bool lane_offsets_fit(const drf_ctx *c, int layout)
     return max_off < (int64_t(1) << 32);
 }
 
-// One volume-kernel launch at the context's precision.
+// A Runge-Kutta step of the volume kernel: the scheme's EpiMode and
+// coefficients (Epi).
+struct StepCoefs {
+    int mode, nst;
+    double c1[kMaxStages], c2[kMaxStages], c3[kMaxStages], q[kMaxStages];
+    const double *dtp;
+};
+
+// One volume-kernel launch at the context's precision: the right-hand side of
+// U into R, or with step the state after a step (R may be U).
 // faces: the context precision's VolFaces (the fused conforming face term
 // of the plain RHS) or null.
-drf_status volume(drf_ctx *c, const void *U, int layout, int mode, int acc_mode, void *R,
-                  const void *U0, void *Y, void *A, const void *X, double c0, double c1,
-                  double c2, double c3, hipStream_t s, const double *dtp = nullptr,
-                  double dtq = 1.0, const void *faces = nullptr)
+template <class T>
+hipError_t volume_t(drf_ctx *c, const void *U, void *R, int layout, hipStream_t s,
+                    const StepCoefs *step, const VolFaces<T> *faces, const T *h, const T *f,
+                    hipError_t (*launch)(int, const VolGeom<T> &, const Ops &, const Phys &,
+                                         View<const T>, const Epi<T> &, hipStream_t))
+{
+    Epi<T> epi{};
+    epi.mode = EPI_RHS;
+    epi.R = view<T>(R, layout, c);
+    if (step) {
+        epi.mode = step->mode;
+        epi.nst = step->nst;
+        for (int k = 0; k < kMaxStages; ++k) {
+            epi.c1[k] = step->c1[k];
+            epi.c2[k] = step->c2[k];
+            epi.c3[k] = step->c3[k];
+            epi.q[k] = step->q[k];
+        }
+        epi.dtp = step->dtp;
+    }
+    VolGeom<T> geo{c->E, coef_view<T>(h, c), coef_view<T>(f, c),
+                   c->f0, c->wg_per_cu, c->xcd_remap, c->wg_lines};
+    if (faces)
+        geo.faces = *faces;
+    return launch(c->order, geo, c->ops, c->phys, cview<T>(U, layout, c), epi, s);
+}
+
+drf_status volume(drf_ctx *c, const void *U, void *R, int layout, hipStream_t s,
+                  const StepCoefs *step = nullptr, const void *faces = nullptr)
 {
     DRF_REQUIRE(lane_offsets_fit(c, layout), DRF_ERR_UNSUPPORTED,
                 "mesh too large for 32-bit per-field offsets in this layout (use LINES or SOA)");
-    hipError_t err;
-    if (c->precision == DRF_PREC_FP64) {
-        Epi<double> epi{};
-        epi.mode = mode;
-        epi.acc_mode = acc_mode;
-        epi.R = view<double>(R, layout, c);
-        epi.U0 = cview<double>(U0, layout, c);
-        epi.Y = view<double>(Y, layout, c);
-        epi.A = view<double>(A, layout, c);
-        epi.X = cview<double>(X, layout, c);
-        epi.c0 = c0;
-        epi.c1 = c1;
-        epi.c2 = c2;
-        epi.c3 = c3;
-        epi.dtp = dtp;
-        epi.dtq = dtq;
-        VolGeom<double> geo{c->E, coef_view<double>(c->d_h, c), coef_view<double>(c->d_f, c),
-                            c->f0, c->wg_per_cu, c->xcd_remap, c->wg_lines};
-        if (faces)
-            geo.faces = *(const VolFaces<double> *)faces;
-        err = launch_volume_fp64(c->order, geo, c->ops, c->phys, cview<double>(U, layout, c), epi,
-                                 s);
-    } else {
-        Epi<float> epi{};
-        epi.mode = mode;
-        epi.acc_mode = acc_mode;
-        epi.R = view<float>(R, layout, c);
-        epi.U0 = cview<float>(U0, layout, c);
-        epi.Y = view<float>(Y, layout, c);
-        epi.A = view<float>(A, layout, c);
-        epi.X = cview<float>(X, layout, c);
-        epi.c0 = c0;
-        epi.c1 = c1;
-        epi.c2 = c2;
-        epi.c3 = c3;
-        epi.dtp = dtp;
-        epi.dtq = dtq;
-        VolGeom<float> geo{c->E, coef_view<float>(c->d_h32, c), coef_view<float>(c->d_f32, c),
-                           c->f0, c->wg_per_cu, c->xcd_remap, c->wg_lines};
-        if (faces)
-            geo.faces = *(const VolFaces<float> *)faces;
-        err = launch_volume_fp32(c->order, geo, c->ops, c->phys, cview<float>(U, layout, c), epi,
-                                 s);
-    }
+    const hipError_t err =
+        c->precision == DRF_PREC_FP64
+            ? volume_t<double>(c, U, R, layout, s, step, (const VolFaces<double> *)faces, c->d_h,
+                               c->d_f, launch_volume_fp64)
+            : volume_t<float>(c, U, R, layout, s, step, (const VolFaces<float> *)faces, c->d_h32,
+                              c->d_f32, launch_volume_fp32);
     if (err != hipSuccess)
         return fail(DRF_ERR_HIP, std::string("volume kernel launch: ") + hipGetErrorString(err));
     return DRF_OK;
@@ -208,8 +204,7 @@ drf_status rhs_into(drf_ctx *c, const void *U, void *R, int layout, hipStream_t 
                                         : volume_faces<float>(c->faces, layout, &f32));
     const void *vf = !fused ? nullptr : c->precision == DRF_PREC_FP64 ? (const void *)&f64
                                                                        : (const void *)&f32;
-    drf_status st = volume(c, U, layout, EPI_RHS, 0, R, nullptr, nullptr, nullptr, nullptr, 0, 0,
-                           0, 0, s, nullptr, 1.0, vf);
+    drf_status st = volume(c, U, R, layout, s, nullptr, vf);
     if (st || !c->faces)
         return st;
     return fused ? face_term_mortars(c->faces, U, R, layout, s) : face_term(c->faces, U, R, layout, s);
@@ -334,7 +329,7 @@ drf_status rk_unfused(drf_ctx *c, int scheme, double dt, double *U, int layout, 
     return DRF_OK;
 }
 
-// Fused stepping: each stage's vector update runs in the RHS kernel epilogue.
+// Fused stepping: one launch runs every stage of the step, in place.
 // Every dt-proportional coefficient is (m dt) / q; with dtp (device dt) the
 // kernel forms it from *dtp with the same operations, so both give the same
 // bits for the same dt.
@@ -349,53 +344,53 @@ drf_status rk_fused(drf_ctx *c, int scheme, double dt, void *U, int layout, hipS
             return fail(DRF_ERR_UNSUPPORTED, "device time steps need a fused scheme (not DP45)");
         return rk_unfused(c, scheme, dt, (double *)U, layout, s);
     }
-    const int64_t len = state_len(c, layout);
-    const size_t es = elem_size(c);
-    drf_status st = ensure_work(c, es * len * 2);
-    if (st)
-        return st;
-    char *w = (char *)c->d_work;
-    void *Ut = w, *A = w + es * len;
-    // coefficient m dt / q: its value (host dt) or its multiplier (device dt)
-    auto D = [&](double m, double q) { return dtp ? m : (m * dt) / q; };
-    auto V = [&](const void *Uin, int mode, int acc, const void *U0, void *Y, void *Acc,
-                 const void *X, double c0, double c1, double c2, double c3, double q) {
-        return volume(c, Uin, layout, mode, acc, nullptr, U0, Y, Acc, X, c0, c1, c2, c3, s, dtp,
-                      q);
+    StepCoefs k{};
+    k.dtp = dtp;
+    // appends a stage whose dt coefficient is m dt / q
+    auto stage = [&](double m, double q, double c2, double c3) {
+        k.c1[k.nst] = dtp ? m : (m * dt) / q;
+        k.q[k.nst] = q;
+        k.c2[k.nst] = c2;
+        k.c3[k.nst] = c3;
+        ++k.nst;
     };
     switch (scheme) {
     case DRF_RK_EULER:
-        TRY(V(U, EPI_STAGE, 0, U, U, nullptr, nullptr, 0, D(1.0, 1.0), 0, 0, 1.0));
+        k.mode = EPI_STAGE;
+        stage(1.0, 1.0, 0, 0);
         break;
     case DRF_RK_RK2:
-        TRY(V(U, EPI_STAGE, 0, U, Ut, nullptr, nullptr, 0, D(0.5, 1.0), 0, 0, 1.0));
-        TRY(V(Ut, EPI_STAGE, 0, U, U, nullptr, nullptr, 0, D(1.0, 1.0), 0, 0, 1.0));
+        k.mode = EPI_STAGE;
+        stage(0.5, 1.0, 0, 0);
+        stage(1.0, 1.0, 0, 0);
         break;
     case DRF_RK_SSPRK3:
-        TRY(V(U, EPI_STAGE, 0, U, Ut, nullptr, nullptr, 0, D(1.0, 1.0), 0, 0, 1.0));
-        TRY(V(Ut, EPI_COMB, 0, U, Ut, nullptr, Ut, 0.75, 0.25, D(1.0, 1.0), 0, 1.0));
-        TRY(V(Ut, EPI_COMB, 0, U, U, nullptr, Ut, 1.0 / 3.0, 2.0 / 3.0, D(1.0, 1.0), 0, 1.0));
+        k.mode = EPI_SSP3;
+        stage(1.0, 1.0, 0, 0);
+        stage(1.0, 1.0, 0.75, 0.25);
+        stage(1.0, 1.0, 1.0 / 3.0, 2.0 / 3.0);
         break;
     case DRF_RK_RK4:
-        TRY(V(U, EPI_STAGE, 1, U, Ut, A, nullptr, 0, D(0.5, 1.0), 0, 0, 1.0));
-        TRY(V(Ut, EPI_STAGE_ACC, 0, U, Ut, A, nullptr, 0, D(0.5, 1.0), 2.0, 0, 1.0));
-        TRY(V(Ut, EPI_STAGE_ACC, 0, U, Ut, A, nullptr, 0, D(1.0, 1.0), 2.0, 0, 1.0));
-        TRY(V(Ut, EPI_RK4FIN, 0, U, U, A, nullptr, 0, D(1.0, 6.0), 0, 0, 6.0));
+        k.mode = EPI_RK4;
+        stage(0.5, 1.0, 1.0, 0);
+        stage(0.5, 1.0, 2.0, 0);
+        stage(1.0, 1.0, 2.0, 0);
+        stage(1.0, 6.0, 1.0, 0);
         break;
     case DRF_RK_LSRK45: {
         static const double Ac[5] = {0.0, -0.4178904745, -1.192151694643, -1.697784692471,
                                      -1.514183444257};
         static const double Bc[5] = {0.1496590219993, 0.3792103129999, 0.8229550293869,
                                      0.6994504559488, 0.1530572479681};
-        for (int k = 0; k < 5; ++k)
-            TRY(V(U, EPI_LSRK, k == 0 ? 1 : 2, nullptr, U, A, U, 0, D(1.0, 1.0), Ac[k], Bc[k],
-                  1.0));
+        k.mode = EPI_LSRK;
+        for (int i = 0; i < 5; ++i)
+            stage(1.0, 1.0, Ac[i], Bc[i]);
         break;
     }
     default:
         return fail(DRF_ERR_ARG, "unknown Runge-Kutta scheme " + std::to_string(scheme));
     }
-    return DRF_OK;
+    return volume(c, U, U, layout, s, &k);
 }
 
 drf_status wave_speed(drf_ctx *c, const void *U, int layout, double *out, hipStream_t s)
@@ -1051,7 +1046,7 @@ drf_status drf_graph_rk_adaptive(drf_ctx *c, int scheme, double cfl, double dx_m
     st = ensure_red(c, std::min<int64_t>(2048, (c->E + 3) / 4) + 1);
     if (st)
         return st;
-    return capture_graph(c, elem_size(c) * state_len(c, layout) * 2, n_steps, out, [&](hipStream_t cs) {
+    return capture_graph(c, 0, n_steps, out, [&](hipStream_t cs) {
         return adaptive_step(c, scheme, cfl, dx_min, dt_min, dt_max, U, layout,
                              (double *)dt_dev, (double *)time_dev, cs);
     });
@@ -1073,8 +1068,7 @@ drf_status drf_graph_rk(drf_ctx *c, int scheme, double dt, void *U, int layout, 
     DRF_REQUIRE(fused || c->precision == DRF_PREC_FP64, DRF_ERR_UNSUPPORTED,
                 "un-fused stepping is the FP64 baseline only");
     const bool uses_lincomb = !fused || scheme == DRF_RK_DP45;
-    const size_t bytes = uses_lincomb ? sizeof(double) * state_len(c, layout) * 7
-                                      : elem_size(c) * state_len(c, layout) * 2;
+    const size_t bytes = uses_lincomb ? sizeof(double) * state_len(c, layout) * 7 : 0;
     return capture_graph(c, bytes, n_steps, out, [&](hipStream_t cs) {
         return fused ? rk_fused(c, scheme, dt, U, layout, cs)
                      : rk_unfused(c, scheme, dt, (double *)U, layout, cs);

@@ -141,30 +141,30 @@ inline int64_t layout_state_len(int layout, int64_t E, int n, int nfields)
     return E * nfields * nd;
 }
 
-// Epilogue of the volume kernel: what is done with the tendency k of each node.
+// What the volume kernel does with the tendency k of each node: writes it, or
+// runs a whole Runge-Kutta step.  The right-hand side is element-local, so a
+// step's stages need nothing from other elements: the stage state y and
+// the accumulator a (0 at first) stay in registers from the first stage to the
+// last, and a step reads the state from memory and writes it once.
 enum EpiMode : int {
-    EPI_RHS = 0,       // R = k
-    EPI_STAGE = 1,     // Y = U0 + c1 k ; acc_mode 1 also writes A = k
-    EPI_STAGE_ACC = 2, // A = A + c2 k ; Y = U0 + c1 k
-    EPI_RK4FIN = 3,    // Y = U0 + c1 (A + k)
-    EPI_COMB = 4,      // Y = c0 U0 + c1 (X + c2 k), X = the RHS input state
-    EPI_LSRK = 5,      // A = c2 A + c1 k (acc_mode 1: A = c1 k) ; Y = X + c3 A
+    EPI_RHS = 0,   // R = k
+    EPI_STAGE = 1, // y = u0 + c1 k (Euler, RK2)
+    EPI_SSP3 = 2,  // y = u0 + c1 k, then y = c2 u0 + c3 (y + c1 k)
+    EPI_RK4 = 3,   // a = a + c2 k; y = u0 + c1 k, last u0 + c1 a
+    EPI_LSRK = 4,  // a = c2 a + c1 k; y = y + c3 a
 };
+
+constexpr int kMaxStages = 5;
 
 template <class T> struct Epi {
     int mode;
-    int acc_mode;
-    View<T> R;        // EPI_RHS output
-    View<const T> U0; // base state
-    View<T> Y;        // stage output
-    View<T> A;        // accumulator
-    View<const T> X;  // RHS input state (re-read in the epilogue)
-    double c0, c1, c2, c3;
-    // Device time step: when dtp is set, the stage's dt-proportional
-    // coefficient (c2 of EPI_COMB, c1 otherwise) holds a multiplier m and
-    // becomes (m * dt) / dtq with dt = *dtp, the host's arithmetic.
+    int nst;   // stages of a step
+    View<T> R; // the tendency, or the state after the step (may be the input)
+    double c1[kMaxStages], c2[kMaxStages], c3[kMaxStages];
+    // Device time step: when dtp is set, c1 holds a multiplier m and becomes
+    // (m * dt) / q with dt = *dtp, the host's arithmetic.
     const double *dtp;
-    double dtq;
+    double q[kMaxStages];
 };
 
 // The conforming face term fused into the volume kernel's last phase (a
@@ -220,7 +220,7 @@ inline hipError_t launch_volume_fp64(int order, const VolGeom<double> &geo, cons
                                    const Phys &ph, View<const double> U, const Epi<double> &epi,
                                    hipStream_t s)
 {
-    switch (order <= 4 ? geo.wg_lines : 128) {
+    switch (order <= 4 && epi.mode == EPI_RHS ? geo.wg_lines : 128) {
     case 256: return launch_volume_fp64_w256(order, geo, ops, ph, U, epi, s);
     case 512: return launch_volume_fp64_w512(order, geo, ops, ph, U, epi, s);
     default: return launch_volume_fp64_w128(order, geo, ops, ph, U, epi, s);
@@ -231,7 +231,7 @@ inline hipError_t launch_volume_fp32(int order, const VolGeom<float> &geo, const
                                    const Phys &ph, View<const float> U, const Epi<float> &epi,
                                    hipStream_t s)
 {
-    switch (order <= 4 ? geo.wg_lines : 128) {
+    switch (order <= 4 && epi.mode == EPI_RHS ? geo.wg_lines : 128) {
     case 256: return launch_volume_fp32_w256(order, geo, ops, ph, U, epi, s);
     case 512: return launch_volume_fp32_w512(order, geo, ops, ph, U, epi, s);
     default: return launch_volume_fp32_w128(order, geo, ops, ph, U, epi, s);

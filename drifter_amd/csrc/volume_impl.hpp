@@ -53,12 +53,9 @@ template <int N, int LW> struct Cfg {
     static constexpr int NT = EPB * n2;
     static constexpr int BLOCK = ((NT + 63) / 64) * 64;
     // minimum waves per SIMD the register allocation must allow
-    // (the low-storage stage carries two operand arrays through the
-    // epilogue and gets one wave less)
     template <class TS, int EPI> static constexpr int wpe()
     {
-        const int w = sizeof(TS) == 8 ? (N <= 4 ? 2 : 1) : (N <= 4 ? 3 : 2);
-        return (EPI == EPI_LSRK && w > 1) ? w - 1 : w;
+        return sizeof(TS) == 8 ? (N <= 4 ? 2 : 1) : (N <= 4 ? 3 : 2);
     }
 };
 
@@ -81,18 +78,9 @@ template <class TS, class TC> __device__ __forceinline__ TC ldo(const TS *ubase,
 {
     return (TC)(*(const TS *)((const char *)ubase + off));
 }
-// NT: a streaming (non-temporal) store.  The fused Runge-Kutta stages use it
-// for Y and A: their stores then leave the read-only stage operands (U0)
-// in the last-level cache (RK4 step 739 -> 684 us at 64x64x8, N = 4).  The
-// plain RHS keeps ordinary stores (streaming ones measured 1 % slower when
-// its input comes from HBM).
-template <class TS, bool NT = false>
-__device__ __forceinline__ void sto(TS *ubase, uint32_t off, TS v)
+template <class TS> __device__ __forceinline__ void sto(TS *ubase, uint32_t off, TS v)
 {
-    if constexpr (NT)
-        __builtin_nontemporal_store(v, (TS *)((char *)ubase + off));
-    else
-        *(TS *)((char *)ubase + off) = v;
+    *(TS *)((char *)ubase + off) = v;
 }
 // Byte offsets of (element, line) pairs.  32-bit arithmetic is exact: the
 // host checks that every offset of the launch fits in 32 bits.
@@ -160,27 +148,21 @@ __device__ __forceinline__ void d2line(const TC *__restrict__ D, const TC *__res
 // The state lines a thread needs for phase P1, with the Coriolis parameter
 // along the line (a field, or the constant f0).
 template <int n, class TC> struct Lines {
-    TC hu[n], hv[n], et[n], ht[n], hs[n], hb[n], fc[n];
+    TC q[5][n]; // Hu, Hv, eta, HT, HS
+    TC hb[n], fc[n];
 };
 
-// All of P1's global loads are issued here, so that P1 itself waits only for
-// them: a load issued inside P1 would make the wave wait for every store of
-// the previous batch as well (gfx9 counts loads and stores in one in-order
-// counter).
-template <int n, int EPB, class TS, class TC>
-__device__ __forceinline__ void load_lines(Lines<n, TC> &L, const View<const TS> &U,
-                                           const VolGeom<TS> &geo, int64_t b, int64_t e, int line)
+template <int n, class TS, class TC>
+__device__ __forceinline__ void load_h(Lines<n, TC> &L, const VolGeom<TS> &geo, int64_t e, int line)
 {
-    const uint32_t uo = state_off<EPB>(U, b, e, line), ho = flat_off(geo.h, e, line);
+    const uint32_t ho = flat_off(geo.h, e, line);
 #pragma unroll
-    for (int i = 0; i < n; ++i) {
-        L.hu[i] = ldo<TS, TC>(U.p + 0 * U.fs + i * U.is, uo);
-        L.hv[i] = ldo<TS, TC>(U.p + 1 * U.fs + i * U.is, uo);
-        L.et[i] = ldo<TS, TC>(U.p + 2 * U.fs + i * U.is, uo);
-        L.ht[i] = ldo<TS, TC>(U.p + 3 * U.fs + i * U.is, uo);
-        L.hs[i] = ldo<TS, TC>(U.p + 4 * U.fs + i * U.is, uo);
+    for (int i = 0; i < n; ++i)
         L.hb[i] = ldo<TS, TC>(geo.h.p + i * geo.h.is, ho);
-    }
+}
+template <int n, class TS, class TC>
+__device__ __forceinline__ void load_f(Lines<n, TC> &L, const VolGeom<TS> &geo, int64_t e, int line)
+{
     if (geo.f.p) {
         const uint32_t fo = flat_off(geo.f, e, line);
 #pragma unroll
@@ -193,73 +175,107 @@ __device__ __forceinline__ void load_lines(Lines<n, TC> &L, const View<const TS>
     }
 }
 
+// All of P1's global loads are issued here, so that P1 itself waits only for
+// them: a load issued inside P1 would make the wave wait for every store of
+// the previous batch as well (gfx9 counts loads and stores in one in-order
+// counter).
+template <int n, int EPB, bool WITH_F, class TS, class TC>
+__device__ __forceinline__ void load_lines(Lines<n, TC> &L, const View<const TS> &U,
+                                           const VolGeom<TS> &geo, int64_t b, int64_t e, int line)
+{
+    const uint32_t uo = state_off<EPB>(U, b, e, line);
+#pragma unroll
+    for (int i = 0; i < n; ++i) {
+#pragma unroll
+        for (int f = 0; f < 5; ++f)
+            L.q[f][i] = ldo<TS, TC>(U.p + f * U.fs + i * U.is, uo);
+    }
+    load_h<n, TS, TC>(L, geo, e, line);
+    if (WITH_F)
+        load_f<n, TS, TC>(L, geo, e, line);
+}
+
 constexpr int kXcds = 8; // MI355X: 8 XCDs of 32 CUs
 
-// Writes fields [F0, F0 + NFD) of the thread's xi-line: the tendency k (RHS)
-// or a fused Runge-Kutta stage update, whose operand lines are loaded here,
-// field by field, right before they are combined.  so: the line's byte
-// offset in every state view (state_off).
-template <int n, int F0, int NFD, class TS, class TC, int EPI>
-__device__ __forceinline__ void write_fields(const Epi<TS> &epi, uint32_t so,
+// Writes fields [F0, F0 + NFD) of the thread's xi-line.  so: the line's byte
+// offset in the state views (state_off).
+template <int n, int F0, int NFD, class TS, class TC>
+__device__ __forceinline__ void write_fields(const View<TS> &R, uint32_t so,
                                              const TC (&kv)[NFD][n])
 {
-    double d1 = epi.c1, d2 = epi.c2;
-    if (EPI != EPI_RHS && epi.dtp) { // dt from device memory (adaptive stepping)
-        const double dt = *epi.dtp;
-        if (EPI == EPI_COMB)
-            d2 = (d2 * dt) / epi.dtq;
-        else
-            d1 = (d1 * dt) / epi.dtq;
-    }
-    const TC c0 = (TC)epi.c0, c1 = (TC)d1, c2 = (TC)d2, c3 = (TC)epi.c3;
-    if (EPI == EPI_RHS) {
-        const uint32_t ro = so;
 #pragma unroll
-        for (int f = 0; f < NFD; ++f)
+    for (int f = 0; f < NFD; ++f)
 #pragma unroll
-            for (int i = 0; i < n; ++i)
-                sto<TS>(epi.R.p + (F0 + f) * epi.R.fs + i * epi.R.is, ro, (TS)kv[f][i]);
-        return;
-    }
-    const View<const TS> V1 = (EPI == EPI_LSRK) ? epi.X : epi.U0;
-    const View<const TS> V2 = (EPI == EPI_COMB)
-                                  ? epi.X
-                                  : View<const TS>{epi.A.p, epi.A.fs, epi.A.es, epi.A.ls,
-                                                   epi.A.is, epi.A.bs, epi.A.bb};
-    const bool two = (EPI == EPI_STAGE_ACC || EPI == EPI_RK4FIN || EPI == EPI_COMB ||
-                      (EPI == EPI_LSRK && epi.acc_mode != 1));
-    const uint32_t q1 = so, q2 = so, yo = so, ao = so;
+        for (int i = 0; i < n; ++i)
+            sto<TS>(R.p + (F0 + f) * R.fs + i * R.is, so, (TS)kv[f][i]);
+}
+
+// What the schemes read of the thread's xi-line besides the tendency: the
+// step's initial state, which is U until the step's own stores and is read
+// again (from the L2) a phase before each use, and an accumulator, which stays
+// in registers.  (With the initial state in registers too, FP64 at N = 4
+// spilled 48 VGPRs per lane.)
+constexpr bool step_reads_u0(int epi) { return epi != EPI_RHS && epi != EPI_LSRK; }
+constexpr bool step_has_acc(int epi) { return epi == EPI_RK4 || epi == EPI_LSRK; }
+
+// Fields [F0, F0 + NFD) of the xi-line at offset so
+template <int n, int F0, int NFD, class TS, class TC>
+__device__ __forceinline__ void load_fields(const View<const TS> &U, uint32_t so,
+                                            TC (&u)[NFD][n])
+{
 #pragma unroll
-    for (int f = 0; f < NFD; ++f) {
-        TC o1[n], o2[n];
+    for (int f = 0; f < NFD; ++f)
+#pragma unroll
+        for (int i = 0; i < n; ++i)
+            u[f][i] = ldo<TS, TC>(U.p + (F0 + f) * U.fs + i * U.is, so);
+}
+
+// The coefficients of one stage (EpiMode), the dt-proportional one formed from
+// the device dt in adaptive steps.
+template <class TC> struct StageCoefs {
+    TC c1, c2, c3;
+    bool first, last;
+};
+template <class TS, class TC>
+__device__ __forceinline__ StageCoefs<TC> stage_coefs(const Epi<TS> &epi, int st)
+{
+    double d = epi.c1[st];
+    if (epi.dtp)
+        d = (d * *epi.dtp) / epi.q[st];
+    return {(TC)d, (TC)epi.c2[st], (TC)epi.c3[st], st == 0, st == epi.nst - 1};
+}
+
+// Fields [F0, F0 + NFD) of the stage state y after a stage with tendency k
+// and initial state u0, with the association of the reference's stage sums.
+// acc is 0 before the first stage.  First and last stages differ by selects:
+// branches on them, one per value, cost registers and time.
+template <int n, int F0, int NFD, int EPI, int NA, class TC>
+__device__ __forceinline__ void stage_update(const StageCoefs<TC> &c, const TC (&k)[NFD][n],
+                                             const TC (&u0)[NFD][n], TC (&y)[5][n],
+                                             TC (&acc)[NA][n])
+{
+#pragma unroll
+    for (int f = 0; f < NFD; ++f)
 #pragma unroll
         for (int i = 0; i < n; ++i) {
-            o1[i] = ldo<TS, TC>(V1.p + (F0 + f) * V1.fs + i * V1.is, q1);
-            o2[i] = two ? ldo<TS, TC>(V2.p + (F0 + f) * V2.fs + i * V2.is, q2) : (TC)0;
-        }
-#pragma unroll
-        for (int i = 0; i < n; ++i) {
-            const TC k = kv[f][i];
-            TC y;
-            if (EPI == EPI_STAGE) { // Y = U0 + c1 k ; A = k (acc_mode 1)
-                if (epi.acc_mode == 1)
-                    sto<TS, true>(epi.A.p + (F0 + f) * epi.A.fs + i * epi.A.is, ao, (TS)k);
-                y = o1[i] + c1 * k;
-            } else if (EPI == EPI_STAGE_ACC) { // A = A + c2 k ; Y = U0 + c1 k
-                sto<TS, true>(epi.A.p + (F0 + f) * epi.A.fs + i * epi.A.is, ao, (TS)(o2[i] + c2 * k));
-                y = o1[i] + c1 * k;
-            } else if (EPI == EPI_RK4FIN) { // Y = U0 + c1 (A + k)
-                y = o1[i] + c1 * (o2[i] + k);
-            } else if (EPI == EPI_COMB) { // Y = c0 U0 + c1 (X + c2 k)
-                y = c0 * o1[i] + c1 * (o2[i] + c2 * k);
-            } else { // EPI_LSRK: A = c2 A + c1 k ; Y = X + c3 A
-                const TC a = (epi.acc_mode == 1) ? c1 * k : c2 * o2[i] + c1 * k;
-                sto<TS, true>(epi.A.p + (F0 + f) * epi.A.fs + i * epi.A.is, ao, (TS)a);
-                y = o1[i] + c3 * a;
+            const TC ki = k[f][i];
+            TC &yi = y[F0 + f][i];
+            if constexpr (EPI == EPI_STAGE) {
+                yi = u0[f][i] + c.c1 * ki;
+            } else if constexpr (EPI == EPI_SSP3) {
+                const TC t = yi + c.c1 * ki; // y is u0 in the first stage
+                const TC r = c.c2 * u0[f][i] + c.c3 * t;
+                yi = c.first ? t : r;
+            } else if constexpr (EPI == EPI_RK4) {
+                TC &a = acc[F0 + f][i]; // c2 = 1, 2, 2, 1
+                a = a + c.c2 * ki;
+                yi = u0[f][i] + c.c1 * (c.last ? a : ki);
+            } else if constexpr (EPI == EPI_LSRK) {
+                TC &a = acc[F0 + f][i]; // c2 = 0 first
+                a = c.c2 * a + c.c1 * ki;
+                yi = yi + c.c3 * a;
             }
-            sto<TS, true>(epi.Y.p + (F0 + f) * epi.Y.fs + i * epi.Y.is, yo, (TS)y);
         }
-    }
 }
 
 // The conforming face term of one element's xi-line, added to the line of
@@ -355,7 +371,17 @@ __device__ __forceinline__ void face_phase(const VolFaces<TS> &fc, const View<co
 // The kernel.  Seven LDS slots per element node, six of them reused in two
 // rounds (momentum, then tracers), so a workgroup of 5 N=4 elements needs
 // 35 KB of staging plus 4 KB of column integrals, and the CU's occupancy is
-// set by registers (4 workgroups at N=4 FP64) rather than by LDS:
+// set by registers (4 workgroups at N=4 FP64) rather than by LDS.
+//
+// With EPI a step's scheme, the phases below run once per stage on a batch
+// whose state never leaves the registers: memory sees the state read and
+// written once per step and, each stage, the batch's own lines of U and h
+// again, which the L2 still holds (about 100 KB per CU).  One launch per
+// stage, each streaming the state and its operands, was bound by HBM at
+// 10 GB per RK4 step of 262,144 FP32 N=4 elements; here the bound is the
+// VALU and the LDS.  RK4, N=4: FP64 32,768 elements 640 -> 200 us, FP32
+// 262,144 elements 2,950 -> 815 us; SSP-RK3, FP64, N=3, 4,096 elements
+// 35.8 -> 21.8 us (one launch in place of three).
 //
 //   P1  xi-owner   xi-derivatives of the momentum terms (registers), column
 //                  integrals (FP64), stages A=Hu v, B=Hv v, C=eta, D=u, E=v, F=H,
@@ -374,9 +400,11 @@ __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_wav
                   const View<const TS> U, const Epi<TS> epi, const int64_t nbatch)
 {
     using C = Cfg<N, LW>;
-    // Fused stages load their operand lines in the epilogue; the next-batch
-    // prefetch is kept for the plain RHS, where registers allow it.
-    constexpr bool PREFETCH = EPI == EPI_RHS;
+    // The right-hand side prefetches the next batch's lines.  A Runge-Kutta
+    // step keeps its stage state, initial state and accumulator in those
+    // registers instead, and runs every stage of one batch before the next.
+    constexpr bool STEP = EPI != EPI_RHS;
+    constexpr bool PREFETCH = !STEP;
     constexpr int n = C::n, n2 = C::n2, n3 = C::n3, EPB = C::EPB;
     __shared__ TC sm[EPB][S_NF][n3];
     // column integrals, double-buffered by batch parity: the last phase of
@@ -389,24 +417,23 @@ __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_wav
     // FACES: face-rule weight by face DOF and M^-1 by node
     __shared__ TS sWq[FACES ? n2 : 1], sMinv[FACES ? n3 : 1];
 
-    // The plain RHS runs every lane through every phase, so that no phase
-    // sits behind an exec-mask branch: lanes past the tile repeat the last
-    // line of the last element (in the same wavefront, in lockstep), and
-    // elements past the end of the mesh repeat element E - 1 in their own LDS
-    // slots.  Their stores write the values the owners write.  With the
+    // Every lane runs through every phase, so that no phase sits behind an
+    // exec-mask branch: lanes past the tile repeat the last line of the last
+    // element (in the same wavefront, in lockstep), and elements past the end
+    // of the mesh repeat element E - 1 in their own LDS slots.  Their stores
+    // of the right-hand side write the values the owners write.  With the
     // stores on every path, P1 waits only for the prefetched lines and not
-    // for the previous batch's stores to drain.  The fused stages, whose
-    // epilogues read and rewrite their accumulators, mask such lanes.
-    constexpr bool DUP = PREFETCH;
+    // for the previous batch's stores to drain.  A step, which rewrites its
+    // input in place, stores from the owners only (what the other lanes read
+    // may already be the new state; nothing of theirs is kept).
     const int tid = threadIdx.x;
-    const bool in_tile = DUP || tid < C::NT;
-    const int tq = (DUP && tid >= C::NT) ? C::NT - 1 : tid;
-    const int le = in_tile ? tq / n2 : 0;
-    const int L = in_tile ? tq - le * n2 : 0;
+    const int tq = tid >= C::NT ? C::NT - 1 : tid;
+    const int le = tq / n2;
+    const int L0 = tq - le * n2;
     const int64_t elast = geo.E - 1;
     auto elem = [&](int64_t bb) {
         const int64_t x = bb * EPB + le;
-        return (DUP && x > elast) ? elast : x;
+        return x > elast ? elast : x;
     };
 
     const TC g = (TC)ph.g, nu_h = (TC)ph.nu_h, nu_v = (TC)ph.nu_v, kT = (TC)ph.kT, kS = (TC)ph.kS;
@@ -444,38 +471,60 @@ __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_wav
     Lines<n, TC> nxt;
     if (PREFETCH) {
         const int64_t e0 = elem(b);
-        if (in_tile && b < nbatch && e0 < geo.E)
-            load_lines<n, EPB, TS, TC>(nxt, U, geo, b, e0, L);
+        if (b < nbatch && e0 < geo.E)
+            load_lines<n, EPB, PREFETCH, TS, TC>(nxt, U, geo, b, e0, L0);
     }
 
-    for (int par = 0; b < nbatch; b += G, par ^= 1) {
+    int par = 0;
+    for (; b < nbatch; b += G) {
         const int64_t e = elem(b);
-        const bool act = DUP || (in_tile && e < geo.E);
-        // With the prefetch, P1 reads the prefetched lines in place (the
-        // next batch's loads overwrite them only after P1's barrier), so the
-        // loop carries no register copies that would wait for those loads.
-        Lines<n, TC> own;
-        if (!PREFETCH && act)
-            load_lines<n, EPB, TS, TC>(own, U, geo, b, e, L);
-        const Lines<n, TC> &cur = PREFETCH ? nxt : own;
-        TC *s = &sm[le][0][0];
+        // P1 reads the prefetched lines in place (the next batch's loads
+        // overwrite them only after P1's barrier), so the loop carries no
+        // register copies that would wait for those loads.  In a step, nxt
+        // is the stage state.
+        if (STEP)
+            load_lines<n, EPB, PREFETCH, TS, TC>(nxt, U, geo, b, e, L0);
+        Lines<n, TC> &cur = nxt;
+        TC acc[step_has_acc(EPI) ? 5 : 1][n];
+        if constexpr (step_has_acc(EPI)) {
+#pragma unroll
+            for (int f = 0; f < 5; ++f)
+#pragma unroll
+                for (int i = 0; i < n; ++i)
+                    acc[f][i] = (TC)0;
+        }
+        // One evaluation of the right-hand side of cur (a lambda and no loop
+        // around the phases for the plain right-hand side: a loop of one trip
+        // cost it 35 VGPRs at N = 3).
+        auto evaluate = [&](int st) __attribute__((always_inline)) {
+        // In a step the line is opaque to the compiler, so that it hoists no
+        // load or address out of the stages into registers they do not have.
+        int L = L0;
+        if constexpr (STEP)
+            asm volatile("" : "+v"(L));
+        // nodes of the xi-, eta- and zeta-line in slot 0
+        TC *const s = &sm[le][0][0];
+        TC *sx = s + L * n, *sy = s + L % n + L / n * n2, *sz = s + L;
+        const StageCoefs<TC> sc = stage_coefs<TS, TC>(epi, st);
 
         // Register state carried by the xi-owner: the momentum partials
         // (P1 -> P4a), HT and HS (P1 -> P4a), the tracer partials (P4a -> P4b).
         TC pHu[n], pHv[n], ht[n], hs[n];
 
         // ---------------- P1: xi-line (j, k) = (L % n, L / n) ----------------
-        if (act) {
+        if constexpr (STEP)
+            load_f<n, TS, TC>(nxt, geo, e, L);
+        {
             TC H[n], u[n], v[n], hinv[n];
 #pragma unroll
             for (int i = 0; i < n; ++i) {
-                H[i] = cur.et[i] + cur.hb[i];
+                H[i] = cur.q[2][i] + cur.hb[i];
                 hinv[i] = hinv_of(H[i]);
                 const TC hi = hinv[i];
-                u[i] = cur.hu[i] * hi;
-                v[i] = cur.hv[i] * hi;
-                ht[i] = cur.ht[i];
-                hs[i] = cur.hs[i];
+                u[i] = cur.q[0][i] * hi;
+                v[i] = cur.q[1][i] * hi;
+                ht[i] = cur.q[3][i];
+                hs[i] = cur.q[4][i];
             }
             // xi-derivatives (momentum_advection :275-305,
             // barotropic_pressure_gradient :322-337, horizontal_diffusion
@@ -483,19 +532,19 @@ __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_wav
             TC x[n], d[n];
 #pragma unroll
             for (int i = 0; i < n; ++i)
-                x[i] = cur.hu[i] * u[i];
+                x[i] = cur.q[0][i] * u[i];
             dline<n>(D, x, d);
 #pragma unroll
             for (int i = 0; i < n; ++i)
-                pHu[i] = -d[i] + cur.fc[i] * cur.hv[i];
+                pHu[i] = -d[i] + cur.fc[i] * cur.q[1][i];
 #pragma unroll
             for (int i = 0; i < n; ++i)
-                x[i] = cur.hv[i] * u[i];
+                x[i] = cur.q[1][i] * u[i];
             dline<n>(D, x, d);
 #pragma unroll
             for (int i = 0; i < n; ++i)
-                pHv[i] = -d[i] + (-cur.fc[i]) * cur.hu[i];
-            dline<n>(D, cur.et, d);
+                pHv[i] = -d[i] + (-cur.fc[i]) * cur.q[0][i];
+            dline<n>(D, cur.q[2], d);
 #pragma unroll
             for (int i = 0; i < n; ++i)
                 pHu[i] += (-g * H[i]) * d[i];
@@ -509,22 +558,21 @@ __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_wav
                 pHv[i] += H[i] * (nu_h * d[i]);
 #pragma unroll
             for (int i = 0; i < n; ++i) {
-                const int m = L * n + i;
-                s[S_A * n3 + m] = cur.hu[i] * v[i];
-                s[S_B * n3 + m] = cur.hv[i] * v[i];
-                s[S_C * n3 + m] = cur.et[i];
-                s[S_D * n3 + m] = u[i];
-                s[S_E * n3 + m] = v[i];
-                s[S_F * n3 + m] = H[i];
-                s[S_G * n3 + m] = hinv[i];
+                sx[S_A * n3 + i] = cur.q[0][i] * v[i];
+                sx[S_B * n3 + i] = cur.q[1][i] * v[i];
+                sx[S_C * n3 + i] = cur.q[2][i];
+                sx[S_D * n3 + i] = u[i];
+                sx[S_E * n3 + i] = v[i];
+                sx[S_F * n3 + i] = H[i];
+                sx[S_G * n3 + i] = hinv[i];
             }
             // Column integrals of compute_eta_rhs (:244-254): over the xi index,
             // summed in node order from 0, in FP64 at every precision.
             double su = 0.0, sv = 0.0;
 #pragma unroll
             for (int i = 0; i < n; ++i) {
-                su += ops.sw[i] * (double)cur.hu[i];
-                sv += ops.sw[i] * (double)cur.hv[i];
+                su += ops.sw[i] * (double)cur.q[0][i];
+                sv += ops.sw[i] * (double)cur.q[1][i];
             }
             bar[par][le][0][L] = su;
             bar[par][le][1][L] = sv;
@@ -539,24 +587,22 @@ __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_wav
             // does not interleave its arithmetic with these loads (6 (N + 1)
             // per lane; 1 % on the FP64 and mixed RHS at 128x128x16, N = 4)
             __builtin_amdgcn_s_setprio(2);
-            if (in_tile && bn < nbatch && en < geo.E)
-                load_lines<n, EPB, TS, TC>(nxt, U, geo, bn, en, L);
+            if (bn < nbatch && en < geo.E)
+                load_lines<n, EPB, PREFETCH, TS, TC>(nxt, U, geo, bn, en, L);
             __builtin_amdgcn_s_setprio(0);
         }
 
         // ---------------- P2a: eta-line (i, k) = (L % n, L / n) ----------------
-        if (act) {
-            const int i0 = L % n, k0 = L / n;
+        {
             TC fuv[n], fvv[n], et[n], u[n], v[n], H[n];
 #pragma unroll
             for (int j = 0; j < n; ++j) {
-                const int m = i0 + n * j + n2 * k0;
-                fuv[j] = s[S_A * n3 + m];
-                fvv[j] = s[S_B * n3 + m];
-                et[j] = s[S_C * n3 + m];
-                u[j] = s[S_D * n3 + m];
-                v[j] = s[S_E * n3 + m];
-                H[j] = s[S_F * n3 + m];
+                fuv[j] = sy[S_A * n3 + j * n];
+                fvv[j] = sy[S_B * n3 + j * n];
+                et[j] = sy[S_C * n3 + j * n];
+                u[j] = sy[S_D * n3 + j * n];
+                v[j] = sy[S_E * n3 + j * n];
+                H[j] = sy[S_F * n3 + j * n];
             }
             TC d[n], aHu[n], aHv[n];
             dline<n>(D, fuv, d);
@@ -581,54 +627,56 @@ __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_wav
                 aHv[j] += H[j] * (nu_h * d[j]);
 #pragma unroll
             for (int j = 0; j < n; ++j) {
-                const int m = i0 + n * j + n2 * k0;
-                s[S_A * n3 + m] = aHu[j];
-                s[S_B * n3 + m] = aHv[j];
+                sy[S_A * n3 + j * n] = aHu[j];
+                sy[S_B * n3 + j * n] = aHv[j];
             }
         }
         __syncthreads();
 
         // ---------------- P3a: zeta-line (i, j) = L, momentum ----------------
-        if (act) {
+        TC um[2][n]; // initial Hu, Hv for P4a
+        if constexpr (step_reads_u0(EPI))
+            load_fields<n, 0, 2>(U, state_off<EPB>(U, b, e, L), um);
+        {
             TC u[n], v[n], hi[n];
 #pragma unroll
             for (int k = 0; k < n; ++k) {
-                const int m = L + n2 * k;
-                u[k] = s[S_D * n3 + m];
-                v[k] = s[S_E * n3 + m];
-                hi[k] = s[S_G * n3 + m];
+                u[k] = sz[S_D * n3 + k * n2];
+                v[k] = sz[S_E * n3 + k * n2];
+                hi[k] = sz[S_G * n3 + k * n2];
             }
             // vertical_diffusion :357-375: nu_v * d2/dzeta2 * Hinv
             TC d[n];
             d2line<n>(D, D2, u, d);
 #pragma unroll
             for (int k = 0; k < n; ++k)
-                s[S_A * n3 + L + n2 * k] += nu_v * d[k] * hi[k];
+                sz[S_A * n3 + k * n2] += nu_v * d[k] * hi[k];
             d2line<n>(D, D2, v, d);
 #pragma unroll
             for (int k = 0; k < n; ++k)
-                s[S_B * n3 + L + n2 * k] += nu_v * d[k] * hi[k];
+                sz[S_B * n3 + k * n2] += nu_v * d[k] * hi[k];
         }
         __syncthreads();
 
         // ---------------- P4a: xi-line again: momentum done, tracers staged ----------------
         TC pHT[n], pHS[n];
-        if (act) {
+        {
             TC kv[2][n];
 #pragma unroll
             for (int i = 0; i < n; ++i) {
-                const int m = L * n + i;
-                kv[0][i] = pHu[i] + s[S_A * n3 + m];
-                kv[1][i] = pHv[i] + s[S_B * n3 + m];
+                kv[0][i] = pHu[i] + sx[S_A * n3 + i];
+                kv[1][i] = pHv[i] + sx[S_B * n3 + i];
             }
-            write_fields<n, 0, 2, TS, TC, EPI>(epi, state_off<EPB>(U, b, e, L), kv);
+            if constexpr (STEP)
+                stage_update<n, 0, 2, EPI>(sc, kv, um, cur.q, acc);
+            else
+                write_fields<n, 0, 2, TS, TC>(epi.R, state_off<EPB>(U, b, e, L), kv);
             TC u[n], v[n], hi[n];
 #pragma unroll
             for (int i = 0; i < n; ++i) {
-                const int m = L * n + i;
-                u[i] = s[S_D * n3 + m];
-                v[i] = s[S_E * n3 + m];
-                hi[i] = s[S_G * n3 + m];
+                u[i] = sx[S_D * n3 + i];
+                v[i] = sx[S_E * n3 + i];
+                hi[i] = sx[S_G * n3 + i];
             }
             // tracer_advection :377-393 along xi
             TC x[n], d[n];
@@ -648,11 +696,10 @@ __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_wav
                 pHS[i] = -d[i];
 #pragma unroll
             for (int i = 0; i < n; ++i) {
-                const int m = L * n + i;
-                s[S_A * n3 + m] = v[i] * ht[i];
-                s[S_B * n3 + m] = v[i] * hs[i];
-                s[S_C * n3 + m] = ht[i] * hi[i];
-                s[S_D * n3 + m] = hs[i] * hi[i];
+                sx[S_A * n3 + i] = v[i] * ht[i];
+                sx[S_B * n3 + i] = v[i] * hs[i];
+                sx[S_C * n3 + i] = ht[i] * hi[i];
+                sx[S_D * n3 + i] = hs[i] * hi[i];
             }
         }
         __syncthreads();
@@ -661,46 +708,47 @@ __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_wav
         // Both roles in one phase: the eta-owner reads and rewrites A, B along
         // its eta-line, the zeta-owner C, D along its zeta-line, so no two
         // threads touch the same node of the same slot.
-        if (act) {
-            const int i0 = L % n, k0 = L / n;
+        TC ut[3][n]; // initial eta, HT, HS for P4b
+        if constexpr (step_reads_u0(EPI))
+            load_fields<n, 2, 3>(U, state_off<EPB>(U, b, e, L), ut);
+        {
             TC ftv[n], fsv[n];
 #pragma unroll
             for (int j = 0; j < n; ++j) {
-                const int m = i0 + n * j + n2 * k0;
-                ftv[j] = s[S_A * n3 + m];
-                fsv[j] = s[S_B * n3 + m];
+                ftv[j] = sy[S_A * n3 + j * n];
+                fsv[j] = sy[S_B * n3 + j * n];
             }
             TC dT[n], dS[n];
             dline<n>(D, ftv, dT);
             dline<n>(D, fsv, dS);
 #pragma unroll
             for (int j = 0; j < n; ++j) {
-                const int m = i0 + n * j + n2 * k0;
-                s[S_A * n3 + m] = -dT[j];
-                s[S_B * n3 + m] = -dS[j];
+                sy[S_A * n3 + j * n] = -dT[j];
+                sy[S_B * n3 + j * n] = -dS[j];
             }
             TC T[n], S[n], hi[n];
 #pragma unroll
             for (int k = 0; k < n; ++k) {
-                const int m = L + n2 * k;
-                T[k] = s[S_C * n3 + m];
-                S[k] = s[S_D * n3 + m];
-                hi[k] = s[S_G * n3 + m];
+                T[k] = sz[S_C * n3 + k * n2];
+                S[k] = sz[S_D * n3 + k * n2];
+                hi[k] = sz[S_G * n3 + k * n2];
             }
             TC d[n];
             d2line<n>(D, D2, T, d);
 #pragma unroll
             for (int k = 0; k < n; ++k)
-                s[S_C * n3 + L + n2 * k] = kT * d[k] * hi[k];
+                sz[S_C * n3 + k * n2] = kT * d[k] * hi[k];
             d2line<n>(D, D2, S, d);
 #pragma unroll
             for (int k = 0; k < n; ++k)
-                s[S_D * n3 + L + n2 * k] = kS * d[k] * hi[k];
+                sz[S_D * n3 + k * n2] = kS * d[k] * hi[k];
         }
         __syncthreads();
 
         // ---------------- P4b: xi-line: free surface and tracers done ----------------
-        if (act) {
+        if constexpr (STEP)
+            load_h<n, TS, TC>(nxt, geo, e, L); // for the next stage's P1
+        {
             const int j0 = L % n, k0 = L / n;
             // eta tendency (:256-272): -(D_x2d HU_bar + D_y2d HV_bar), where the
             // 2D "x" index is j and the 2D "y" index is k.
@@ -714,12 +762,14 @@ __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_wav
             TC kv[3][n];
 #pragma unroll
             for (int i = 0; i < n; ++i) {
-                const int m = L * n + i;
                 kv[0][i] = deta;
-                kv[1][i] = (pHT[i] + s[S_A * n3 + m]) + s[S_C * n3 + m];
-                kv[2][i] = (pHS[i] + s[S_B * n3 + m]) + s[S_D * n3 + m];
+                kv[1][i] = (pHT[i] + sx[S_A * n3 + i]) + sx[S_C * n3 + i];
+                kv[2][i] = (pHS[i] + sx[S_B * n3 + i]) + sx[S_D * n3 + i];
             }
-            write_fields<n, 2, 3, TS, TC, EPI>(epi, state_off<EPB>(U, b, e, L), kv);
+            if constexpr (STEP)
+                stage_update<n, 2, 3, EPI>(sc, kv, ut, cur.q, acc);
+            else
+                write_fields<n, 2, 3, TS, TC>(epi.R, state_off<EPB>(U, b, e, L), kv);
         }
         // ---------------- P5 (FACES): the conforming face term ----------------
         // Not by the lanes that repeat element E - 1 from another wavefront:
@@ -729,8 +779,20 @@ __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_wav
                 face_phase<n, TS>(geo.faces, U, epi.R, e, L, sWq, sMinv);
         }
         // No barrier here: this phase reads only its own line's slots and the
-        // column integrals of this batch's parity; the next batch's P1 writes
-        // its own line's slots and the other parity.
+        // column integrals of this parity; the next P1 (of the next stage or
+        // batch) writes its own line's slots and the other parity.
+        par ^= 1;
+        };
+        if constexpr (STEP) {
+#pragma unroll 1
+            for (int st = 0; st < epi.nst; ++st)
+                evaluate(st);
+        } else {
+            evaluate(0);
+        }
+        if constexpr (STEP)
+            if (tid < C::NT && b * EPB + le < geo.E)
+                write_fields<n, 0, 5, TS, TC>(epi.R, state_off<EPB>(U, b, e, L0), cur.q);
     }
 }
 
@@ -786,15 +848,23 @@ hipError_t launch_ne(const VolGeom<TS> &geo, const Ops &ops, const Phys &ph, Vie
             v = 1;
         return v;
     }();
-    // persistent workgroups: a few rounds per workgroup so the next batch's
-    // loads overlap the current batch's arithmetic
-    const int wpc = (geo.wg_per_cu > 0 && geo.wg_per_cu < per_cu) ? geo.wg_per_cu : per_cu;
-    if (EPI == EPI_RHS) // what a requested shape amounts to, for the autotuner's report
+    int64_t grid = nbatch;
+    if (EPI == EPI_RHS) {
+        // persistent workgroups: a few rounds per workgroup so the next batch's
+        // loads overlap the current batch's arithmetic
+        const int wpc = (geo.wg_per_cu > 0 && geo.wg_per_cu < per_cu) ? geo.wg_per_cu : per_cu;
+        // what a requested shape amounts to, for the autotuner's report
         g_rhs_per_cu[sizeof(TS) == 8 ? 0 : 1][LW == 128 ? 0 : LW == 256 ? 1 : 2][N][FACES] =
             per_cu;
-    int64_t grid = (int64_t)num_cus() * wpc;
-    if (grid > nbatch)
-        grid = nbatch;
+        grid = (int64_t)num_cus() * wpc;
+        if (grid > nbatch)
+            grid = nbatch;
+    } else {
+        // a step has nothing to prefetch: one batch per workgroup, so that the
+        // last round is balanced by the hardware; whole rounds of the XCDs for
+        // the batch order
+        grid = (nbatch + kXcds - 1) / kXcds * kXcds;
+    }
     hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(C::BLOCK), 0, s, geo,
                        make_ops<N + 1, TC>(ops), ph, U, epi, nbatch);
     return hipGetLastError();
@@ -807,15 +877,17 @@ hipError_t launch_n(const VolGeom<TS> &geo, const Ops &ops, const Phys &ph, View
     if constexpr (N <= 4) // face plans are built for orders 1-4
         if (epi.mode == EPI_RHS && geo.faces.eface)
             return launch_ne<N, TS, TC, EPI_RHS, LW, true>(geo, ops, ph, U, epi, s);
-    switch (epi.mode) {
-    case EPI_RHS: return launch_ne<N, TS, TC, EPI_RHS, LW, false>(geo, ops, ph, U, epi, s);
-    case EPI_STAGE: return launch_ne<N, TS, TC, EPI_STAGE, LW, false>(geo, ops, ph, U, epi, s);
-    case EPI_STAGE_ACC: return launch_ne<N, TS, TC, EPI_STAGE_ACC, LW, false>(geo, ops, ph, U, epi, s);
-    case EPI_RK4FIN: return launch_ne<N, TS, TC, EPI_RK4FIN, LW, false>(geo, ops, ph, U, epi, s);
-    case EPI_COMB: return launch_ne<N, TS, TC, EPI_COMB, LW, false>(geo, ops, ph, U, epi, s);
-    case EPI_LSRK: return launch_ne<N, TS, TC, EPI_LSRK, LW, false>(geo, ops, ph, U, epi, s);
-    default: return hipErrorInvalidValue;
-    }
+    if (epi.mode == EPI_RHS)
+        return launch_ne<N, TS, TC, EPI_RHS, LW, false>(geo, ops, ph, U, epi, s);
+    if constexpr (LW == 128) // whole steps
+        switch (epi.mode) {
+        case EPI_STAGE: return launch_ne<N, TS, TC, EPI_STAGE, LW, false>(geo, ops, ph, U, epi, s);
+        case EPI_SSP3: return launch_ne<N, TS, TC, EPI_SSP3, LW, false>(geo, ops, ph, U, epi, s);
+        case EPI_RK4: return launch_ne<N, TS, TC, EPI_RK4, LW, false>(geo, ops, ph, U, epi, s);
+        case EPI_LSRK: return launch_ne<N, TS, TC, EPI_LSRK, LW, false>(geo, ops, ph, U, epi, s);
+        default: break;
+        }
+    return hipErrorInvalidValue;
 }
 
 // Orders above 4 run at 128 lines per workgroup only: their registers exceed

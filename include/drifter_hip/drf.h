@@ -153,8 +153,8 @@ drf_status drf_autotune(drf_ctx *ctx, const void *U, void *dUdt, int layout, int
 
 /* One step of `scheme` on the host packed state U (in/out). */
 drf_status drf_rk_step(drf_ctx *ctx, int scheme, double t, double dt, double *U);
-/* Device-resident state; fused != 0 fuses the stage updates into the RHS
- * kernel epilogue, fused == 0 runs the reference's sequence (RHS, then
+/* Device-resident state; fused != 0 runs every stage of the step in one
+ * kernel (DP45 excepted), fused == 0 runs the reference's sequence (RHS, then
  * separate vector updates). */
 drf_status drf_rk_step_dev(drf_ctx *ctx, int scheme, double t, double dt, void *U, int layout,
                            int fused, void *stream);

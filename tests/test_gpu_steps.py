@@ -1,0 +1,89 @@
+"""Whole Runge-Kutta steps in one launch (the volume kernel's step modes)
+against the same scheme composed of right-hand sides and vector updates, at
+every order, precision and layout, on element counts around one workgroup's
+batch (128 grid lines: 128 // (N + 1)^2 elements) and past it.
+
+Tolerance: both sides evaluate the same expressions; they differ in FMA
+contraction only.  Each stage's combination rounds a few times at the size of
+the state (8 eps of the field's maximum covers five stages), and a tendency's
+rounding enters multiplied by dt (a contraction of n terms of operands up to
+the largest |D| ~ n^2: 1e-12 of the largest tendency in FP64, 1e-4 in FP32).
+"""
+import numpy as np
+import pytest
+
+from drifter_amd import _lib, synth
+from drifter_amd.solver import CoriolisParameter, PrimitiveEquationsSolver
+
+pytestmark = pytest.mark.gpu
+
+SCHEMES = {"euler": _lib.RK_EULER, "rk2": _lib.RK_RK2, "ssprk3": _lib.RK_SSPRK3,
+           "rk4": _lib.RK_RK4, "lsrk45": _lib.RK_LSRK45}
+LAYOUTS = (_lib.LAYOUT_PACKED, _lib.LAYOUT_SOA, _lib.LAYOUT_LINES, _lib.LAYOUT_BLOCKS)
+
+
+def _composed(k, U, scheme, dt):
+    if scheme == "euler":
+        return U + dt * k(U)
+    if scheme == "rk2":
+        return U + dt * k(U + (0.5 * dt) * k(U))
+    if scheme == "ssprk3":
+        a = U + dt * k(U)
+        b = 0.75 * U + 0.25 * (a + dt * k(a))
+        return (1.0 / 3.0) * U + (2.0 / 3.0) * (b + dt * k(b))
+    if scheme == "rk4":
+        k1 = k(U)
+        k2 = k(U + (0.5 * dt) * k1)
+        k3 = k(U + (0.5 * dt) * k2)
+        return U + (dt / 6.0) * (((k1 + 2.0 * k2) + 2.0 * k3) + k(U + dt * k3))
+    A = (0.0, -0.4178904745, -1.192151694643, -1.697784692471, -1.514183444257)
+    B = (0.1496590219993, 0.3792103129999, 0.8229550293869, 0.6994504559488, 0.1530572479681)
+    Y, r = U, 0.0 * U
+    for a, b in zip(A, B):
+        r = a * r + dt * k(Y)
+        Y = Y + b * r
+    return Y
+
+
+@pytest.mark.parametrize("order", range(1, 9))
+@pytest.mark.parametrize("prec", [_lib.PREC_FP64, _lib.PREC_MIXED])
+@pytest.mark.parametrize("scheme", sorted(SCHEMES))
+def test_step_is_the_composed_scheme(order, prec, scheme):
+    import torch
+
+    n = order + 1
+    batch = max(1, 128 // (n * n))
+    full = synth.make_case(5, 5, 8, order, 10000.0, "seamount")
+    nd, dtype = n ** 3, torch.float64 if prec == _lib.PREC_FP64 else torch.float32
+    eps = float(np.finfo(np.float64 if prec == _lib.PREC_FP64 else np.float32).eps)
+    dt = 1e-3
+    for q, E in enumerate(sorted({1, max(1, batch - 1), batch, batch + 1, 3 * batch + 2})):
+        E = min(E, full.E)
+        layout = LAYOUTS[(q + order) % 4]
+        print(f"[step] order={order} prec={prec} {scheme} E={E} layout={layout}", flush=True)
+        s = PrimitiveEquationsSolver(order, prec)
+        beta = 2e-11 if q % 2 else 0.0
+        s.initialize(E, full.h[:E * nd], coriolis=CoriolisParameter(1e-4, beta, 0.0),
+                     y_positions=full.y[:E * nd])
+        P = full.U[:E * 5 * nd]
+        if layout == _lib.LAYOUT_SOA:
+            P = synth.to_soa(P, E, nd)
+        elif layout == _lib.LAYOUT_LINES:
+            P = synth.to_lines(P, E, n)
+        elif layout == _lib.LAYOUT_BLOCKS:
+            P = synth.to_blocks(P, E, n, _lib.load().drf_layout_block_elements(order))
+        U = torch.from_numpy(np.ascontiguousarray(P)).cuda().to(dtype)
+
+        def k(V):
+            R = torch.zeros_like(V)
+            s.compute_rhs_dev(V.contiguous(), R, layout)
+            return R
+
+        want = _composed(k, U, scheme, dt)
+        rate = float(k(U).abs().max())
+        got = U.clone()
+        s.rk_step_dev(SCHEMES[scheme], 0.0, dt, got, layout)
+        torch.cuda.synchronize()
+        tol = 8 * eps * float(U.abs().max()) + dt * (1e-12 if eps < 1e-12 else 1e-4) * rate
+        assert float((got - want).abs().max()) <= tol
+        s.close()
