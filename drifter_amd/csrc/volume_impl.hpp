@@ -59,6 +59,83 @@ template <int N, int LW> struct Cfg {
     }
 };
 
+// LDS placement of the staged values.  Node (i, j, k) of a slot sits at
+// i + j SJ + k SK, slots SS apart, elements ES apart.  The LDS serves 32 banks
+// of 4 bytes a clock, so B = 32 float or 16 double lanes at a time: SJ, SK and
+// ES (mod B) are such that B consecutive xi-lines lie in distinct banks where
+// some padding can do it (odd n need none, n = 6 in FP64 has no LDS to spare),
+// and the eta- and zeta-lines are dealt to the lanes by line_order, so that
+// theirs do too.  Naturally placed and dealt, the accesses took 3.2 (N = 3),
+// 1.6 (N = 4) and 4.5 (N = 7) times their conflict-free clocks in FP64, and
+// 3.5, 2.0 and 5.0 times in FP32; now 1.0 to 1.3 (n = 2 and FP64 n = 6: 1.5).
+// RK4 of 4 M nodes in FP64: N = 3 205 -> 174 us, N = 4 204 -> 196 us, N = 7
+// 450 -> 405 us; in FP32 N = 3 97.6 -> 88.7 us, N = 4 110.9 -> 100.0 us.
+template <int n, int BYTES> struct Place {
+    static constexpr int B = 128 / BYTES;
+    static constexpr bool D = BYTES == 8;
+    static constexpr int SJ = n == 6 ? (D ? 6 : 7) : n == 8 ? 9 : n;
+    static constexpr int SK = n == 4 ? (D ? 17 : 19) : n == 6 ? (D ? 36 : 42) : n == 8 ? 72 : n * n;
+    // element stride modulo B
+    static constexpr int EM = (n == 2   ? 9
+                               : n == 4 ? (D ? 68 : 80)
+                               : n == 6 ? (D ? 219 : 252)
+                               : n == 8 ? (D ? 584 : 583)
+                                        : n * n * n) % B;
+    static constexpr int SS = (n - 1) * (1 + SJ + SK) + 1;
+    static constexpr int ES = S_NF * SS + (EM + B - S_NF * SS % B) % B;
+};
+
+// The eta- and zeta-lines of a batch in the order the lanes take them: entry t
+// packs the first node's place (element part included) of lane t's eta-line
+// (low half) and zeta-line.  Each group of B lanes takes one line from each of
+// the fullest banks in turn.
+template <int NT> struct LineOrder {
+    uint32_t v[NT];
+};
+template <int n, int EPB, int BYTES> constexpr LineOrder<EPB * n * n> line_order()
+{
+    using P = Place<n, BYTES>;
+    constexpr int NT = EPB * n * n, B = P::B;
+    static_assert(EPB * P::ES < 65536, "line places are packed in 16 bits");
+    LineOrder<NT> r{};
+    for (int z = 0; z < 2; ++z) {
+        int place[NT] = {}, left[B] = {};
+        bool used[NT] = {};
+        for (int t = 0; t < NT; ++t) {
+            const int e = t / (n * n), L = t % (n * n);
+            place[t] = e * P::ES + L % n + (L / n) * (z ? P::SJ : P::SK);
+            ++left[place[t] % B];
+        }
+        int out = 0;
+        while (out < NT) {
+            const int end = out + B < NT ? out + B : NT;
+            while (out < end) {
+                // one pass over the banks, fullest first
+                bool taken[B] = {};
+                for (int pass = 0; pass < B && out < end; ++pass) {
+                    int best = -1;
+                    for (int b = 0; b < B; ++b)
+                        if (!taken[b] && left[b] > 0 && (best < 0 || left[b] > left[best]))
+                            best = b;
+                    if (best < 0)
+                        break;
+                    taken[best] = true;
+                    int t = 0;
+                    while (used[t] || place[t] % B != best)
+                        ++t;
+                    used[t] = true;
+                    --left[best];
+                    r.v[out++] |= (uint32_t)place[t] << (16 * z);
+                }
+            }
+        }
+    }
+    return r;
+}
+template <int n, int EPB, int BYTES> struct LineTable {
+    static constexpr LineOrder<EPB * n * n> order = line_order<n, EPB, BYTES>();
+};
+
 // Operators sized for one order, passed by value (kernel-argument SGPRs).
 template <int n, class TC> struct KOps {
     TC D[n * n];   // 1D derivative matrix, row-major
@@ -379,9 +456,9 @@ __device__ __forceinline__ void face_phase(const VolFaces<TS> &fc, const View<co
 // again, which the L2 still holds (about 100 KB per CU).  One launch per
 // stage, each streaming the state and its operands, was bound by HBM at
 // 10 GB per RK4 step of 262,144 FP32 N=4 elements; here the bound is the
-// VALU and the LDS.  RK4, N=4: FP64 32,768 elements 640 -> 200 us, FP32
-// 262,144 elements 2,950 -> 815 us; SSP-RK3, FP64, N=3, 4,096 elements
-// 35.8 -> 21.8 us (one launch in place of three).
+// VALU and the LDS.  RK4, N=4: FP64 32,768 elements 640 -> 196 us, FP32
+// 262,144 elements 2,950 -> 750 us; SSP-RK3, FP64, N=3, 4,096 elements
+// 35.8 -> 20 us (one launch in place of three).
 //
 //   P1  xi-owner   xi-derivatives of the momentum terms (registers), column
 //                  integrals (FP64), stages A=Hu v, B=Hv v, C=eta, D=u, E=v, F=H,
@@ -405,8 +482,12 @@ __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_wav
     // registers instead, and runs every stage of one batch before the next.
     constexpr bool STEP = EPI != EPI_RHS;
     constexpr bool PREFETCH = !STEP;
+    // FP64 from N = 6 has no registers to load a step's initial state a phase
+    // early (SSP-RK3 at N = 8: 555 us early, 544 us at the use)
+    constexpr bool LATE = sizeof(TC) == 8 && N >= 6;
     constexpr int n = C::n, n2 = C::n2, n3 = C::n3, EPB = C::EPB;
-    __shared__ TC sm[EPB][S_NF][n3];
+    using P = Place<n, (int)sizeof(TC)>;
+    __shared__ TC sm[EPB * P::ES];
     // column integrals, double-buffered by batch parity: the last phase of
     // one batch reads them while the first phase of the next writes
     __shared__ double bar[2][EPB][2][n2];
@@ -430,6 +511,8 @@ __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_wav
     const int tq = tid >= C::NT ? C::NT - 1 : tid;
     const int le = tq / n2;
     const int L0 = tq - le * n2;
+    // first nodes of this lane's eta- and zeta-line
+    const uint32_t lines = LineTable<n, EPB, (int)sizeof(TC)>::order.v[tq];
     const int64_t elast = geo.E - 1;
     auto elem = [&](int64_t bb) {
         const int64_t x = bb * EPB + le;
@@ -503,8 +586,8 @@ __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_wav
         if constexpr (STEP)
             asm volatile("" : "+v"(L));
         // nodes of the xi-, eta- and zeta-line in slot 0
-        TC *const s = &sm[le][0][0];
-        TC *sx = s + L * n, *sy = s + L % n + L / n * n2, *sz = s + L;
+        TC *sx = sm + le * P::ES + (L % n) * P::SJ + (L / n) * P::SK;
+        TC *sy = sm + (lines & 0xffffu), *sz = sm + (lines >> 16);
         const StageCoefs<TC> sc = stage_coefs<TS, TC>(epi, st);
 
         // Register state carried by the xi-owner: the momentum partials
@@ -558,13 +641,13 @@ __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_wav
                 pHv[i] += H[i] * (nu_h * d[i]);
 #pragma unroll
             for (int i = 0; i < n; ++i) {
-                sx[S_A * n3 + i] = cur.q[0][i] * v[i];
-                sx[S_B * n3 + i] = cur.q[1][i] * v[i];
-                sx[S_C * n3 + i] = cur.q[2][i];
-                sx[S_D * n3 + i] = u[i];
-                sx[S_E * n3 + i] = v[i];
-                sx[S_F * n3 + i] = H[i];
-                sx[S_G * n3 + i] = hinv[i];
+                sx[S_A * P::SS + i] = cur.q[0][i] * v[i];
+                sx[S_B * P::SS + i] = cur.q[1][i] * v[i];
+                sx[S_C * P::SS + i] = cur.q[2][i];
+                sx[S_D * P::SS + i] = u[i];
+                sx[S_E * P::SS + i] = v[i];
+                sx[S_F * P::SS + i] = H[i];
+                sx[S_G * P::SS + i] = hinv[i];
             }
             // Column integrals of compute_eta_rhs (:244-254): over the xi index,
             // summed in node order from 0, in FP64 at every precision.
@@ -597,12 +680,12 @@ __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_wav
             TC fuv[n], fvv[n], et[n], u[n], v[n], H[n];
 #pragma unroll
             for (int j = 0; j < n; ++j) {
-                fuv[j] = sy[S_A * n3 + j * n];
-                fvv[j] = sy[S_B * n3 + j * n];
-                et[j] = sy[S_C * n3 + j * n];
-                u[j] = sy[S_D * n3 + j * n];
-                v[j] = sy[S_E * n3 + j * n];
-                H[j] = sy[S_F * n3 + j * n];
+                fuv[j] = sy[S_A * P::SS + j * P::SJ];
+                fvv[j] = sy[S_B * P::SS + j * P::SJ];
+                et[j] = sy[S_C * P::SS + j * P::SJ];
+                u[j] = sy[S_D * P::SS + j * P::SJ];
+                v[j] = sy[S_E * P::SS + j * P::SJ];
+                H[j] = sy[S_F * P::SS + j * P::SJ];
             }
             TC d[n], aHu[n], aHv[n];
             dline<n>(D, fuv, d);
@@ -627,34 +710,34 @@ __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_wav
                 aHv[j] += H[j] * (nu_h * d[j]);
 #pragma unroll
             for (int j = 0; j < n; ++j) {
-                sy[S_A * n3 + j * n] = aHu[j];
-                sy[S_B * n3 + j * n] = aHv[j];
+                sy[S_A * P::SS + j * P::SJ] = aHu[j];
+                sy[S_B * P::SS + j * P::SJ] = aHv[j];
             }
         }
         __syncthreads();
 
         // ---------------- P3a: zeta-line (i, j) = L, momentum ----------------
         TC um[2][n]; // initial Hu, Hv for P4a
-        if constexpr (step_reads_u0(EPI))
+        if constexpr (step_reads_u0(EPI) && !LATE)
             load_fields<n, 0, 2>(U, state_off<EPB>(U, b, e, L), um);
         {
             TC u[n], v[n], hi[n];
 #pragma unroll
             for (int k = 0; k < n; ++k) {
-                u[k] = sz[S_D * n3 + k * n2];
-                v[k] = sz[S_E * n3 + k * n2];
-                hi[k] = sz[S_G * n3 + k * n2];
+                u[k] = sz[S_D * P::SS + k * P::SK];
+                v[k] = sz[S_E * P::SS + k * P::SK];
+                hi[k] = sz[S_G * P::SS + k * P::SK];
             }
             // vertical_diffusion :357-375: nu_v * d2/dzeta2 * Hinv
             TC d[n];
             d2line<n>(D, D2, u, d);
 #pragma unroll
             for (int k = 0; k < n; ++k)
-                sz[S_A * n3 + k * n2] += nu_v * d[k] * hi[k];
+                sz[S_A * P::SS + k * P::SK] += nu_v * d[k] * hi[k];
             d2line<n>(D, D2, v, d);
 #pragma unroll
             for (int k = 0; k < n; ++k)
-                sz[S_B * n3 + k * n2] += nu_v * d[k] * hi[k];
+                sz[S_B * P::SS + k * P::SK] += nu_v * d[k] * hi[k];
         }
         __syncthreads();
 
@@ -664,9 +747,11 @@ __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_wav
             TC kv[2][n];
 #pragma unroll
             for (int i = 0; i < n; ++i) {
-                kv[0][i] = pHu[i] + sx[S_A * n3 + i];
-                kv[1][i] = pHv[i] + sx[S_B * n3 + i];
+                kv[0][i] = pHu[i] + sx[S_A * P::SS + i];
+                kv[1][i] = pHv[i] + sx[S_B * P::SS + i];
             }
+            if constexpr (step_reads_u0(EPI) && LATE)
+                load_fields<n, 0, 2>(U, state_off<EPB>(U, b, e, L), um);
             if constexpr (STEP)
                 stage_update<n, 0, 2, EPI>(sc, kv, um, cur.q, acc);
             else
@@ -674,9 +759,9 @@ __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_wav
             TC u[n], v[n], hi[n];
 #pragma unroll
             for (int i = 0; i < n; ++i) {
-                u[i] = sx[S_D * n3 + i];
-                v[i] = sx[S_E * n3 + i];
-                hi[i] = sx[S_G * n3 + i];
+                u[i] = sx[S_D * P::SS + i];
+                v[i] = sx[S_E * P::SS + i];
+                hi[i] = sx[S_G * P::SS + i];
             }
             // tracer_advection :377-393 along xi
             TC x[n], d[n];
@@ -696,10 +781,10 @@ __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_wav
                 pHS[i] = -d[i];
 #pragma unroll
             for (int i = 0; i < n; ++i) {
-                sx[S_A * n3 + i] = v[i] * ht[i];
-                sx[S_B * n3 + i] = v[i] * hs[i];
-                sx[S_C * n3 + i] = ht[i] * hi[i];
-                sx[S_D * n3 + i] = hs[i] * hi[i];
+                sx[S_A * P::SS + i] = v[i] * ht[i];
+                sx[S_B * P::SS + i] = v[i] * hs[i];
+                sx[S_C * P::SS + i] = ht[i] * hi[i];
+                sx[S_D * P::SS + i] = hs[i] * hi[i];
             }
         }
         __syncthreads();
@@ -709,45 +794,47 @@ __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_wav
         // its eta-line, the zeta-owner C, D along its zeta-line, so no two
         // threads touch the same node of the same slot.
         TC ut[3][n]; // initial eta, HT, HS for P4b
-        if constexpr (step_reads_u0(EPI))
+        if constexpr (step_reads_u0(EPI) && !LATE)
             load_fields<n, 2, 3>(U, state_off<EPB>(U, b, e, L), ut);
         {
             TC ftv[n], fsv[n];
 #pragma unroll
             for (int j = 0; j < n; ++j) {
-                ftv[j] = sy[S_A * n3 + j * n];
-                fsv[j] = sy[S_B * n3 + j * n];
+                ftv[j] = sy[S_A * P::SS + j * P::SJ];
+                fsv[j] = sy[S_B * P::SS + j * P::SJ];
             }
             TC dT[n], dS[n];
             dline<n>(D, ftv, dT);
             dline<n>(D, fsv, dS);
 #pragma unroll
             for (int j = 0; j < n; ++j) {
-                sy[S_A * n3 + j * n] = -dT[j];
-                sy[S_B * n3 + j * n] = -dS[j];
+                sy[S_A * P::SS + j * P::SJ] = -dT[j];
+                sy[S_B * P::SS + j * P::SJ] = -dS[j];
             }
             TC T[n], S[n], hi[n];
 #pragma unroll
             for (int k = 0; k < n; ++k) {
-                T[k] = sz[S_C * n3 + k * n2];
-                S[k] = sz[S_D * n3 + k * n2];
-                hi[k] = sz[S_G * n3 + k * n2];
+                T[k] = sz[S_C * P::SS + k * P::SK];
+                S[k] = sz[S_D * P::SS + k * P::SK];
+                hi[k] = sz[S_G * P::SS + k * P::SK];
             }
             TC d[n];
             d2line<n>(D, D2, T, d);
 #pragma unroll
             for (int k = 0; k < n; ++k)
-                sz[S_C * n3 + k * n2] = kT * d[k] * hi[k];
+                sz[S_C * P::SS + k * P::SK] = kT * d[k] * hi[k];
             d2line<n>(D, D2, S, d);
 #pragma unroll
             for (int k = 0; k < n; ++k)
-                sz[S_D * n3 + k * n2] = kS * d[k] * hi[k];
+                sz[S_D * P::SS + k * P::SK] = kS * d[k] * hi[k];
         }
         __syncthreads();
 
         // ---------------- P4b: xi-line: free surface and tracers done ----------------
         if constexpr (STEP)
-            load_h<n, TS, TC>(nxt, geo, e, L); // for the next stage's P1
+            // for the next stage's P1, after the last one too: a branch here
+            // keeps the old line alive (RK4, FP64, N = 4: 196 -> 381 us)
+            load_h<n, TS, TC>(nxt, geo, e, L);
         {
             const int j0 = L % n, k0 = L / n;
             // eta tendency (:256-272): -(D_x2d HU_bar + D_y2d HV_bar), where the
@@ -763,9 +850,11 @@ __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_wav
 #pragma unroll
             for (int i = 0; i < n; ++i) {
                 kv[0][i] = deta;
-                kv[1][i] = (pHT[i] + sx[S_A * n3 + i]) + sx[S_C * n3 + i];
-                kv[2][i] = (pHS[i] + sx[S_B * n3 + i]) + sx[S_D * n3 + i];
+                kv[1][i] = (pHT[i] + sx[S_A * P::SS + i]) + sx[S_C * P::SS + i];
+                kv[2][i] = (pHS[i] + sx[S_B * P::SS + i]) + sx[S_D * P::SS + i];
             }
+            if constexpr (step_reads_u0(EPI) && LATE)
+                load_fields<n, 2, 3>(U, state_off<EPB>(U, b, e, L), ut);
             if constexpr (STEP)
                 stage_update<n, 2, 3, EPI>(sc, kv, ut, cur.q, acc);
             else
@@ -860,10 +949,17 @@ hipError_t launch_ne(const VolGeom<TS> &geo, const Ops &ops, const Phys &ph, Vie
         if (grid > nbatch)
             grid = nbatch;
     } else {
-        // a step has nothing to prefetch: one batch per workgroup, so that the
-        // last round is balanced by the hardware; whole rounds of the XCDs for
-        // the batch order
+        // A step has nothing to prefetch: one batch per workgroup, so that the
+        // hardware balances the last round, in whole rounds of the XCDs for the
+        // batch order (against resident workgroups that loop: RK4 with 4 M
+        // nodes, N = 4, FP64 196 and 219 us, FP32 100 and 114 us).  In FP64
+        // from N = 6 the operators no longer fit the SGPRs and a workgroup's
+        // start, which spills them, costs more than the imbalance: N = 6 424
+        // one batch each, 400 us resident, N = 8 695 and 667 us.
         grid = (nbatch + kXcds - 1) / kXcds * kXcds;
+        const int64_t resident = (int64_t)num_cus() * per_cu;
+        if (sizeof(TS) == 8 && N >= 6 && grid > resident)
+            grid = resident;
     }
     hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(C::BLOCK), 0, s, geo,
                        make_ops<N + 1, TC>(ops), ph, U, epi, nbatch);
