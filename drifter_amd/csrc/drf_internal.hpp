@@ -169,13 +169,14 @@ template <class T> struct Epi {
 
 // The conforming face term fused into the volume kernel's last phase (a
 // face plan's element table; eface == nullptr: none).  Per element face:
-// (neighbour << 4) | (neighbour's face << 1) | side, -1 where not conforming.
+// (neighbour << 1) | side, all ones where not conforming (side 0: this element
+// is the interface's left; a conforming neighbour always meets face f with its
+// opposite face f ^ 1).
 template <class T> struct VolFaces {
-    const int64_t *eface;
+    const uint32_t *eface;
     const T *wq; // face-rule weight by face DOF, (N+1)^2 values, 0 past the N-point rule
     T p[4];      // scalar flux parameters (vx, vy, vz, lambda)
     int kind;    // DRF_FLUX_UPWIND or DRF_FLUX_LF_ADV
-    int nq;      // face DOFs that carry the N-point rule
 };
 
 template <class T> struct VolGeom {

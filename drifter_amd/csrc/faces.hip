@@ -93,11 +93,10 @@ __global__ void __launch_bounds__(256)
 
 // The conforming part of the face term, element by element: every interface
 // seen from each of its two elements, so that a thread adds to its own
-// element's nodes only.  eface[6 e + f] = (neighbour << 4) | (neighbour's face
-// << 1) | side for a conforming face (side 0: this element is the
-// interface's left, whose face gives the normal), -1 otherwise; a conforming
-// neighbour always meets the face with its opposite face f ^ 1.  One thread
-// per (element, field, xi-line): it reads and rewrites its line of U and dU
+// element's nodes only.  eface[6 e + f] = (neighbour << 1) | side for a
+// conforming face (side 0: this element is the interface's left, whose face
+// gives the normal), all ones otherwise; a conforming neighbour always meets
+// the face with its opposite face f ^ 1.  One thread per (element, field, xi-line): it reads and rewrites its line of U and dU
 // (contiguous across the workgroup in the LINES layout, each element's block
 // once) and reads the neighbours' nodes on the shared faces.
 // Per node the contributions of the x, y and z faces are summed (in that
@@ -132,7 +131,7 @@ template <class T> __device__ __forceinline__ T ldb(const T *base, uint32_t off)
 
 template <int n, class T>
 __global__ void __launch_bounds__(256)
-    face_elem_kernel(int64_t E, const int64_t *__restrict__ eface, FaceArgs<T> a)
+    face_elem_kernel(int64_t E, const uint32_t *__restrict__ eface, FaceArgs<T> a)
 {
     // one thread per (element, field, xi-line): every load of a thread is
     // issued before its arithmetic, and a workgroup's lanes for one field
@@ -159,11 +158,12 @@ __global__ void __launch_bounds__(256)
         return (uint32_t)((elem_offset(el, a.es, a.bs, a.bb) + (int64_t)line * a.ls) *
                           (int64_t)sizeof(T));
     };
-    auto entry = [&](int64_t v, int line) {
+    constexpr uint32_t none = 0xffffffffu;
+    auto entry = [&](uint32_t v, int line) {
         FaceNb r;
-        r.on = v >= 0;
-        r.side = (int)(v & 1);
-        r.off = r.on ? line_off(v >> 4, line) : 0u;
+        r.on = v != none;
+        r.side = (int)(v & 1u);
+        r.off = r.on ? line_off(v >> 1, line) : 0u;
         return r;
     };
     // the faces this line lies on: both x-faces (its end nodes), a y-face
@@ -185,8 +185,8 @@ __global__ void __launch_bounds__(256)
         if (e >= E)
             continue;
         const FaceNb x0 = entry(eface[6 * e], L), x1 = entry(eface[6 * e + 1], L);
-        const FaceNb y = entry(fy >= 0 ? eface[6 * e + fy] : -1, Ly);
-        const FaceNb z = entry(fz >= 0 ? eface[6 * e + fz] : -1, Lz);
+        const FaceNb y = entry(fy >= 0 ? eface[6 * e + fy] : none, Ly);
+        const FaceNb z = entry(fz >= 0 ? eface[6 * e + fz] : none, Lz);
         const uint32_t own = line_off(e, L);
         T u[n], du[n], ux0 = T(0), ux1 = T(0), uy[n], uz[n];
 #pragma unroll
@@ -236,7 +236,8 @@ __global__ void __launch_bounds__(256)
 // (coarse element, coarse face, fine elements of sub-faces 0..NF-1), the fine
 // faces being the coarse face's opposite.  ops = [Minv | Pc | Lc | Pf[NF] |
 // Lf[NF]] (nm x nm each) of the group's connection type, staged in LDS once
-// per persistent workgroup.  One lane per (interface, field, mortar DOF).
+// per persistent workgroup with rows at an odd stride.  One lane per
+// (interface, field, mortar DOF).
 // LIFT adds M^-1 I^T of rhs_c and rhs_f to the tendencies; otherwise rhs_c
 // is written [m][field][nm] and rhs_f [m][field][NF][nm].
 template <int n, int NF, class T, bool LIFT>
@@ -245,13 +246,14 @@ __global__ void __launch_bounds__(256)
                        const T *__restrict__ ops, FaceArgs<T> a, T *__restrict__ out_c,
                        T *__restrict__ out_f)
 {
-    constexpr int nm = n * n, MM = nm * nm, NMAT = 3 + 2 * NF;
+    // odd row stride of the staged operators
+    constexpr int nm = n * n, RS = nm | 1, MM = nm * RS, NMAT = 3 + 2 * NF;
     constexpr int ipb = 256 / nm;                  // (interface, field) units per pass
     constexpr int per = (1 + NF) * nm + 2 * nm;    // Uc | Uf[NF] | F | M^-1 F
     __shared__ T sops[NMAT * MM];
     __shared__ T sbuf[ipb * per];
-    for (int i = threadIdx.x; i < NMAT * MM; i += blockDim.x)
-        sops[i] = ops[i];
+    for (int i = threadIdx.x; i < NMAT * nm * nm; i += blockDim.x)
+        sops[i / nm * RS + i % nm] = ops[i];
     const T *Minv = sops, *Pc = sops + MM, *Lc = sops + 2 * MM, *Pf = sops + 3 * MM,
             *Lf = sops + (3 + NF) * MM;
     const int g = threadIdx.x / nm, r = threadIdx.x - g * nm;
@@ -268,30 +270,40 @@ __global__ void __launch_bounds__(256)
         const int fc = act ? (int)list[6 * m + 1] : 0, ff = fc ^ 1;
         const int dc = face_node(n, fc, it, jt), df = face_node(n, ff, it, jt);
         const int64_t ec = act ? list[6 * m] : 0;
+        // the tendencies are loaded with the traces: at the lifts their latency
+        // was half the kernel's chain
         int64_t oc = 0, of[NF];
+        T tc = T(0), tf[NF];
         __syncthreads(); // operators staged; the previous units are done with sbuf
         if (act) {
             oc = f * a.fs + node_off(a, n, ec, dc);
             su[r] = a.U[oc];
+            if (LIFT)
+                tc = a.dU[oc];
 #pragma unroll
             for (int k = 0; k < NF; ++k) {
                 of[k] = f * a.fs + node_off(a, n, list[6 * m + 2 + k], df);
                 su[nm + k * nm + r] = a.U[of[k]];
+                if (LIFT)
+                    tf[k] = a.dU[of[k]];
             }
         }
+        const T mc = inv_mass(a, n, dc), mfi = inv_mass(a, n, df);
         __syncthreads();
         if (act) {
             T nrm[3] = {T(0), T(0), T(0)};
             nrm[fc >> 1] = (fc & 1) ? T(1) : T(-1);
             T uc = T(0);
+#pragma unroll
             for (int c = 0; c < nm; ++c)
-                uc += Pc[r * nm + c] * su[c];
+                uc += Pc[r * RS + c] * su[c];
             T uf = T(0);
 #pragma unroll
             for (int k = 0; k < NF; ++k) {
                 T s = T(0);
+#pragma unroll
                 for (int c = 0; c < nm; ++c)
-                    s += Pf[k * MM + r * nm + c] * su[nm + k * nm + c];
+                    s += Pf[k * MM + r * RS + c] * su[nm + k * nm + c];
                 uf += s;
             }
             sF[r] = scalar_flux_t<T>(a.kind, uc, uf, nrm, a.p);
@@ -299,27 +311,29 @@ __global__ void __launch_bounds__(256)
         __syncthreads();
         if (act) {
             T mf = T(0);
+#pragma unroll
             for (int c = 0; c < nm; ++c)
-                mf += Minv[r * nm + c] * sF[c];
+                mf += Minv[r * RS + c] * sF[c];
             sF[nm + r] = mf;
         }
         __syncthreads();
         if (act) {
             T rc = T(0);
+#pragma unroll
             for (int c = 0; c < nm; ++c)
-                rc += Lc[r * nm + c] * sF[nm + c];
+                rc += Lc[r * RS + c] * sF[nm + c];
             if (LIFT)
-                a.dU[oc] += inv_mass(a, n, dc) * rc;
+                a.dU[oc] = tc + mc * rc;
             else
                 out_c[(m * 5 + f) * nm + r] = rc;
-            const T mfi = inv_mass(a, n, df);
 #pragma unroll
             for (int k = 0; k < NF; ++k) {
                 T v = T(0);
+#pragma unroll
                 for (int c = 0; c < nm; ++c)
-                    v += -Lf[k * MM + r * nm + c] * sF[nm + c];
+                    v += -Lf[k * MM + r * RS + c] * sF[nm + c];
                 if (LIFT)
-                    a.dU[of[k]] += mfi * v;
+                    a.dU[of[k]] = tf[k] + mfi * v;
                 else
                     out_f[((m * 5 + f) * NF + k) * nm + r] = v;
             }
@@ -347,7 +361,7 @@ hipError_t conf_n(bool lift, int64_t nif, const int64_t *list, const FaceArgs<T>
 }
 
 template <int n, class T>
-hipError_t elem_n(int64_t E, const int64_t *eface, const FaceArgs<T> &a, hipStream_t s)
+hipError_t elem_n(int64_t E, const uint32_t *eface, const FaceArgs<T> &a, hipStream_t s)
 {
     constexpr int EPB = 256 / (5 * n * n);
     const unsigned g8 = (grid_for(E, EPB, 1u << 20) + 7u) & ~7u; // a multiple of 8
@@ -400,7 +414,7 @@ hipError_t launch_face_conforming(int n, bool lift, int64_t nif, const int64_t *
 }
 
 template <class T>
-hipError_t launch_face_elements(int n, int64_t E, const int64_t *eface, const FaceArgs<T> &a,
+hipError_t launch_face_elements(int n, int64_t E, const uint32_t *eface, const FaceArgs<T> &a,
                                 hipStream_t s)
 {
     if (E <= 0)
@@ -436,9 +450,9 @@ template hipError_t launch_face_conforming<double>(int, bool, int64_t, const int
 template hipError_t launch_face_conforming<float>(int, bool, int64_t, const int64_t *,
                                                   const FaceArgs<float> &, float *, float *,
                                                   hipStream_t);
-template hipError_t launch_face_elements<double>(int, int64_t, const int64_t *,
+template hipError_t launch_face_elements<double>(int, int64_t, const uint32_t *,
                                                  const FaceArgs<double> &, hipStream_t);
-template hipError_t launch_face_elements<float>(int, int64_t, const int64_t *,
+template hipError_t launch_face_elements<float>(int, int64_t, const uint32_t *,
                                                 const FaceArgs<float> &, hipStream_t);
 template hipError_t launch_face_mortar<double>(int, int, bool, int64_t, const int64_t *,
                                                const double *, const FaceArgs<double> &, double *,

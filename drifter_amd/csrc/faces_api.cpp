@@ -41,8 +41,9 @@ struct drf_face_plan {
     std::vector<int> mort_type;
     // [E][6]: (neighbour << 4) | (neighbour's face << 1) | side of every
     // conforming face (side 0: the element is the interface's left), else -1
-    std::vector<int64_t> eface;
-    int64_t *d_conf = nullptr, *d_mort = nullptr, *d_eface = nullptr;
+    std::vector<uint32_t> eface;
+    int64_t *d_conf = nullptr, *d_mort = nullptr;
+    uint32_t *d_eface = nullptr;
     void *d_wq = nullptr;   // face-rule weight by face DOF (plan precision), for the fused phase
     // conforming interfaces: DRF_FACES_BY_INTERFACE, _BY_ELEMENT or _IN_VOLUME
     int conf_mode = DRF_FACES_IN_VOLUME;
@@ -232,10 +233,7 @@ drf_status face_term(const drf_face_plan *p, const void *U, void *dU, int layout
 // do not fit), and the mortar groups on their own.
 template <class T> bool volume_faces(const drf_face_plan *p, int layout, VolFaces<T> *out)
 {
-    // the volume kernel's face phase addresses unblocked states: a blocked
-    // state takes the element-ordered launch after the volume kernel
-    if (p->conf_mode != DRF_FACES_IN_VOLUME || p->conf.empty() || !p->d_wq ||
-        layout == DRF_LAYOUT_BLOCKS)
+    if (p->conf_mode != DRF_FACES_IN_VOLUME || p->conf.empty() || !p->d_wq)
         return false;
     FaceArgs<T> a;
     fill_args<T>(p, a, nullptr, nullptr, layout);
@@ -246,7 +244,6 @@ template <class T> bool volume_faces(const drf_face_plan *p, int layout, VolFace
     for (int i = 0; i < 4; ++i)
         out->p[i] = a.p[i];
     out->kind = p->kind;
-    out->nq = a.nq1 * a.nq1;
     return true;
 }
 template bool volume_faces<double>(const drf_face_plan *, int, VolFaces<double> *);
@@ -386,12 +383,12 @@ drf_status drf_face_plan_create(const drf_ctx *ctx, int64_t n_elem, const double
         }
     }
     if (!p->conf.empty()) {
-        p->eface.assign((size_t)E * 6, -1);
+        p->eface.assign((size_t)E * 6, 0xffffffffu);
         for (size_t c = 0; c < p->conf.size(); c += 4) {
             const int64_t el = p->conf[c], fl = p->conf[c + 1], er = p->conf[c + 2],
                           fr = p->conf[c + 3];
-            p->eface[(size_t)(6 * el + fl)] = (er << 4) | (fr << 1);
-            p->eface[(size_t)(6 * er + fr)] = (el << 4) | (fl << 1) | 1;
+            p->eface[(size_t)(6 * el + fl)] = (uint32_t)er << 1;
+            p->eface[(size_t)(6 * er + fr)] = (uint32_t)el << 1 | 1u;
         }
     }
     drf_status st = hipSetDevice(ctx->device) == hipSuccess

@@ -155,16 +155,20 @@ template <class TS, class TC> __device__ __forceinline__ TC ldo(const TS *ubase,
 {
     return (TC)(*(const TS *)((const char *)ubase + off));
 }
-template <class TS> __device__ __forceinline__ void sto(TS *ubase, uint32_t off, TS v)
+// NT: a streaming store, for a result that nothing reads back soon.
+template <class TS, bool NT = false>
+__device__ __forceinline__ void sto(TS *ubase, uint32_t off, TS v)
 {
-    *(TS *)((char *)ubase + off) = v;
+    if constexpr (NT)
+        __builtin_nontemporal_store(v, (TS *)((char *)ubase + off));
+    else
+        *(TS *)((char *)ubase + off) = v;
 }
 // Byte offsets of (element, line) pairs.  32-bit arithmetic is exact: the
 // host checks that every offset of the launch fits in 32 bits.
 //
 // A view without blocks: the bathymetry and Coriolis lines (always in the
-// line layout, no larger than one field of the state), and the fused face
-// phase (which runs on unblocked states only).
+// line layout, no larger than one field of the state).
 template <class T> __device__ __forceinline__ uint32_t flat_off(const View<T> &v, int64_t e, int L)
 {
     return ((uint32_t)e * (uint32_t)v.es + (uint32_t)L * (uint32_t)v.ls) * (uint32_t)sizeof(T);
@@ -256,7 +260,7 @@ __device__ __forceinline__ void load_f(Lines<n, TC> &L, const VolGeom<TS> &geo, 
 // them: a load issued inside P1 would make the wave wait for every store of
 // the previous batch as well (gfx9 counts loads and stores in one in-order
 // counter).
-template <int n, int EPB, bool WITH_F, class TS, class TC>
+template <int n, int EPB, int NF, bool WITH_F, class TS, class TC>
 __device__ __forceinline__ void load_lines(Lines<n, TC> &L, const View<const TS> &U,
                                            const VolGeom<TS> &geo, int64_t b, int64_t e, int line)
 {
@@ -264,7 +268,7 @@ __device__ __forceinline__ void load_lines(Lines<n, TC> &L, const View<const TS>
 #pragma unroll
     for (int i = 0; i < n; ++i) {
 #pragma unroll
-        for (int f = 0; f < 5; ++f)
+        for (int f = 0; f < NF; ++f)
             L.q[f][i] = ldo<TS, TC>(U.p + f * U.fs + i * U.is, uo);
     }
     load_h<n, TS, TC>(L, geo, e, line);
@@ -276,7 +280,7 @@ constexpr int kXcds = 8; // MI355X: 8 XCDs of 32 CUs
 
 // Writes fields [F0, F0 + NFD) of the thread's xi-line.  so: the line's byte
 // offset in the state views (state_off).
-template <int n, int F0, int NFD, class TS, class TC>
+template <int n, int F0, int NFD, bool NT = false, class TS, class TC>
 __device__ __forceinline__ void write_fields(const View<TS> &R, uint32_t so,
                                              const TC (&kv)[NFD][n])
 {
@@ -284,7 +288,7 @@ __device__ __forceinline__ void write_fields(const View<TS> &R, uint32_t so,
     for (int f = 0; f < NFD; ++f)
 #pragma unroll
         for (int i = 0; i < n; ++i)
-            sto<TS>(R.p + (F0 + f) * R.fs + i * R.is, so, (TS)kv[f][i]);
+            sto<TS, NT>(R.p + (F0 + f) * R.fs + i * R.is, so, (TS)kv[f][i]);
 }
 
 // What the schemes read of the thread's xi-line besides the tendency: the
@@ -355,94 +359,209 @@ __device__ __forceinline__ void stage_update(const StageCoefs<TC> &c, const TC (
         }
 }
 
-// The conforming face term of one element's xi-line, added to the line of
-// the tendencies the thread has just written (the fused form of
-// face_elem_kernel, faces.hip, with the same arithmetic and order: per node
-// the x, y and z contributions summed, then M^-1; each interface with its own
-// left/right flux order).  The thread rereads its own writes, so no barrier
-// is needed.
-template <class T>
-__device__ __forceinline__ T face_contrib_v(int kind, const T *prm, int f, int side, T own,
-                                            T other, T wq)
-{
+// The conforming face term in the plain right-hand side: none, or with one of
+// the scalar fluxes (a template argument: a branch between the two fluxes
+// around the neighbours' nodes spilled them).
+enum : int { FACES_NONE = 0, FACES_LF = 1, FACES_UPWIND = 2 };
+
+// One face of the conforming face term seen from one of its elements, for
+// nodes with the value own here and other across: what face_elem_kernel
+// (faces.hip) adds, bit for bit on finite values.  With the interface's normal
+// n = +-e_axis and F its flux in left/right order, the contribution is +wq F
+// on the left and -wq F on the right; both equal wq times the flux formed with
+// this element's outward normal, since every term only changes sign and sums
+// commute.  (UPWIND at vn = 0 takes the left value.)
+//   LF_ADV  0.5 (vn own + vn other) - 0.5 lambda (other - own), and the
+//           normal's zero components make it NaN where a value is not finite
+//   UPWIND  vn (own or other)
+template <class T, bool LF> struct FaceFlux {
+    T vn, hl;
+    bool take_own;
+    __device__ __forceinline__ FaceFlux(const VolFaces<T> &fc, int axis, bool upper, uint32_t entry)
+    {
+        vn = upper ? fc.p[axis] : -fc.p[axis];
+        hl = T(0.5) * fc.p[3];
+        take_own = (entry & 1u) ? !(vn <= T(0)) : vn >= T(0);
+    }
+    __device__ __forceinline__ T operator()(T own, T other, T wq) const
+    {
 #pragma clang fp contract(off)
-    const int fl = side ? (f ^ 1) : f;
-    T nrm[3] = {T(0), T(0), T(0)};
-    nrm[fl >> 1] = (fl & 1) ? T(1) : T(-1);
-    if (side == 0)
-        return T(0) + wq * scalar_flux_t<T>(kind, own, other, nrm, prm);
-    return T(0) - wq * scalar_flux_t<T>(kind, other, own, nrm, prm);
+        if constexpr (LF) {
+            const T d = other - own;
+            const T F = T(0.5) * (vn * own + vn * other) - hl * d;
+            return wq * __builtin_elementwise_fma(d, T(0), F);
+        }
+        return wq * (vn * (take_own ? own : other));
+    }
+};
+
+// The faces xi-line L lies on: both x-faces at its ends, a y-face when j is 0
+// or N, a z-face when k is 0 or N, as entries of the plan's element table
+// (kNoFace elsewhere).  Of a y- or z-face only the lines with points of the
+// N-point face rule (DOFs it + n jt < nq) are kept.
+constexpr uint32_t kNoFace = 0xffffffffu;
+template <int n> struct FaceLine {
+    static constexpr int nq1 = n <= 2 ? 2 : n - 1, nq = nq1 * nq1;
+    uint32_t x0, x1, y, z;
+    __device__ __forceinline__ void load(const uint32_t *__restrict__ eface, int64_t e, int L)
+    {
+        const int j = L % n, k = L / n;
+        const uint32_t *t = eface + 6 * e;
+        const bool x = L < nq, yb = (j == 0 || j == n - 1) && n * k < nq,
+                   zb = (k == 0 || k == n - 1) && n * j < nq;
+        x0 = x ? t[0] : kNoFace;
+        x1 = x ? t[1] : kNoFace;
+        y = yb ? t[j == 0 ? 2 : 3] : kNoFace;
+        z = zb ? t[k == 0 ? 4 : 5] : kNoFace;
+    }
+};
+
+// Byte offset of line L of the neighbour of a table entry (neighbour << 1 | side)
+template <int N, class T>
+__device__ __forceinline__ uint32_t nb_off(const View<T> &v, uint32_t entry, int L)
+{
+    constexpr uint32_t B = (uint32_t)vol_batch_elements(N, N <= 4 ? 512 : 128);
+    const uint32_t e = entry >> 1;
+    uint32_t base = e * (uint32_t)v.es;
+    if (v.bb) // the blocked layout's block is B elements (layout_strides)
+        base = e / B * (uint32_t)v.bs + e % B * (uint32_t)v.es;
+    return (base + (uint32_t)L * (uint32_t)v.ls) * (uint32_t)sizeof(T);
 }
 
-template <int n, class TS>
-__device__ __forceinline__ void face_phase(const VolFaces<TS> &fc, const View<const TS> &U,
-                                           const View<TS> &R, int64_t e, int L, const TS *sWq,
-                                           const TS *sMinv)
-{
+// The neighbours' nodes of fields [F0, F0 + NFD) across the line's faces
+template <int n, int NFD, class T> struct FaceNodes {
+    T x0[NFD], x1[NFD], y[NFD][n], z[NFD][n];
+    template <int F0>
+    __device__ __forceinline__ void load(const FaceLine<n> &fl, const View<const T> &U, int L)
+    {
+        constexpr int nq = FaceLine<n>::nq;
+        const int j = L % n, k = L / n;
+        auto at = [&](int f, int i, uint32_t off) { return ldo<T, T>(U.p + f * U.fs + i * U.is, off); };
+        if (fl.x0 != kNoFace) {
+            const uint32_t o = nb_off<n - 1>(U, fl.x0, L);
+#pragma unroll
+            for (int f = 0; f < NFD; ++f)
+                x0[f] = at(F0 + f, n - 1, o);
+        }
+        if (fl.x1 != kNoFace) {
+            const uint32_t o = nb_off<n - 1>(U, fl.x1, L);
+#pragma unroll
+            for (int f = 0; f < NFD; ++f)
+                x1[f] = at(F0 + f, 0, o);
+        }
+        if (fl.y != kNoFace) {
+            const uint32_t o = nb_off<n - 1>(U, fl.y, (n - 1 - j) + n * k);
+#pragma unroll
+            for (int f = 0; f < NFD; ++f)
+#pragma unroll
+                for (int i = 0; i < n; ++i)
+                    if (i + n * k < nq)
+                        y[f][i] = at(F0 + f, i, o);
+        }
+        if (fl.z != kNoFace) {
+            const uint32_t o = nb_off<n - 1>(U, fl.z, j + n * (n - 1 - k));
+#pragma unroll
+            for (int f = 0; f < NFD; ++f)
+#pragma unroll
+                for (int i = 0; i < n; ++i)
+                    if (i + n * j < nq)
+                        z[f][i] = at(F0 + f, i, o);
+        }
+    }
+    // out[F0 + f] = M^-1 (x, y and z contributions, summed in that order) of
+    // the own nodes q[F0 + f].  A node that was not loaded is not read.
+    template <int F0, bool LF>
+    __device__ __forceinline__ void contrib(const FaceLine<n> &fl, const VolFaces<T> &fc,
+                                            const T (&q)[5][n], int L, const T *sWq,
+                                            const T *sMinv, T (&out)[5][n]) const
+    {
 #pragma clang fp contract(off)
-    struct Nb {
-        uint32_t off;
-        int side;
-        bool on;
-    };
-    const int j = L % n, k = L / n, nq = fc.nq;
-    // the faces this line lies on, and the neighbour's line across each (as
-    // face_elem_kernel: x-faces at its ends, y / z when j / k is 0 or N)
-    const int fy = (j == 0) ? 2 : (j == n - 1) ? 3 : -1;
-    const int fz = (k == 0) ? 4 : (k == n - 1) ? 5 : -1;
-    const int Ly = (n - 1 - j) + n * k, Lz = j + n * (n - 1 - k);
-    auto entry = [&](int f, int line) {
-        const int64_t v = f >= 0 ? fc.eface[6 * e + f] : -1;
-        Nb r;
-        r.on = v >= 0;
-        r.side = (int)(v & 1);
-        r.off = r.on ? flat_off(U, v >> 4, line) : 0u;
-        return r;
-    };
-    const Nb x0 = entry(0, L), x1 = entry(1, L), y = entry(fy, Ly), z = entry(fz, Lz);
-    const uint32_t ou = flat_off(U, e, L), orr = flat_off(R, e, L);
-#pragma unroll 1
-    for (int fld = 0; fld < 5; ++fld) {
-        const TS *Uf = U.p + fld * U.fs;
-        TS *Rf = R.p + fld * R.fs;
-        TS u[n], du[n], uy[n], uz[n], ux0 = TS(0), ux1 = TS(0), acc[n];
+        constexpr int nq = FaceLine<n>::nq;
+        const int j = L % n, k = L / n;
+#pragma unroll
+        for (int f = 0; f < NFD; ++f)
+#pragma unroll
+            for (int i = 0; i < n; ++i)
+                out[F0 + f][i] = T(0);
+        if (fl.x0 != kNoFace) {
+            const FaceFlux<T, LF> F(fc, 0, false, fl.x0);
+            const T w = sWq[L];
+#pragma unroll
+            for (int f = 0; f < NFD; ++f)
+                out[F0 + f][0] += F(q[F0 + f][0], x0[f], w);
+        }
+        if (fl.x1 != kNoFace) {
+            const FaceFlux<T, LF> F(fc, 0, true, fl.x1);
+            const T w = sWq[L];
+#pragma unroll
+            for (int f = 0; f < NFD; ++f)
+                out[F0 + f][n - 1] += F(q[F0 + f][n - 1], x1[f], w);
+        }
+        if (fl.y != kNoFace) {
+            const FaceFlux<T, LF> F(fc, 1, j != 0, fl.y);
+#pragma unroll
+            for (int i = 0; i < n; ++i)
+                if (i + n * k < nq) {
+                    const T w = sWq[i + n * k];
+#pragma unroll
+                    for (int f = 0; f < NFD; ++f)
+                        out[F0 + f][i] += F(q[F0 + f][i], y[f][i], w);
+                }
+        }
+        if (fl.z != kNoFace) {
+            const FaceFlux<T, LF> F(fc, 2, k != 0, fl.z);
+#pragma unroll
+            for (int i = 0; i < n; ++i)
+                if (i + n * j < nq) {
+                    const T w = sWq[i + n * j];
+#pragma unroll
+                    for (int f = 0; f < NFD; ++f)
+                        out[F0 + f][i] += F(q[F0 + f][i], z[f][i], w);
+                }
+        }
 #pragma unroll
         for (int i = 0; i < n; ++i) {
-            u[i] = ldo<TS, TS>(Uf + i * U.is, ou);
-            du[i] = ldo<TS, TS>(Rf + i * R.is, orr);
-            uy[i] = y.on ? ldo<TS, TS>(Uf + i * U.is, y.off) : TS(0);
-            uz[i] = z.on ? ldo<TS, TS>(Uf + i * U.is, z.off) : TS(0);
-            acc[i] = TS(0);
-        }
-        if (x0.on)
-            ux0 = ldo<TS, TS>(Uf + (n - 1) * U.is, x0.off);
-        if (x1.on)
-            ux1 = ldo<TS, TS>(Uf, x1.off);
-        if (L < nq) {
-            const TS wq = sWq[L];
-            if (x0.on)
-                acc[0] += face_contrib_v<TS>(fc.kind, fc.p, 0, x0.side, u[0], ux0, wq);
-            if (x1.on)
-                acc[n - 1] += face_contrib_v<TS>(fc.kind, fc.p, 1, x1.side, u[n - 1], ux1, wq);
-        }
-        if (y.on) {
+            const T m = sMinv[i + n * L];
 #pragma unroll
-            for (int i = 0; i < n; ++i)
-                if (i + n * k < nq)
-                    acc[i] += face_contrib_v<TS>(fc.kind, fc.p, fy, y.side, u[i], uy[i],
-                                                 sWq[i + n * k]);
+            for (int f = 0; f < NFD; ++f)
+                out[F0 + f][i] = m * out[F0 + f][i];
         }
-        if (z.on) {
+    }
+};
+
+// Fields whose neighbour nodes are in flight at once: all where the registers
+// allow it, else one chunk while the next one loads (39,280 elements: FP64
+// N = 3 all 102, one by one 106 us, N = 4 one by one 206, in twos 220 us; FP32
+// N = 4 in twos 116, one by one 121, all 128 us).
+template <int N, class T> constexpr int face_chunk()
+{
+    return N <= 3 ? 5 : sizeof(T) == 8 ? 1 : 2;
+}
+template <int n, int CH, int F0, bool LF, int NFD, class T>
+__device__ __forceinline__ void face_fields(const FaceNodes<n, NFD, T> &fn, const FaceLine<n> &fl,
+                                            const VolFaces<T> &fc, const View<const T> &U,
+                                            const T (&q)[5][n], int L, const T *sWq,
+                                            const T *sMinv, T (&out)[5][n])
+{
+    constexpr int F1 = F0 + NFD;
+    if constexpr (F1 < 5) {
+        FaceNodes<n, (F1 + CH <= 5 ? CH : 5 - F1), T> next;
+        next.template load<F1>(fl, U, L);
+        fn.template contrib<F0, LF>(fl, fc, q, L, sWq, sMinv, out);
+        face_fields<n, CH, F1, LF>(next, fl, fc, U, q, L, sWq, sMinv, out);
+    } else {
+        fn.template contrib<F0, LF>(fl, fc, q, L, sWq, sMinv, out);
+    }
+}
+
+template <int n, int F0, int NFD, class T>
+__device__ __forceinline__ void add_faces(T (&k)[NFD][n], const T (&fa)[5][n])
+{
 #pragma unroll
-            for (int i = 0; i < n; ++i)
-                if (i + n * j < nq)
-                    acc[i] += face_contrib_v<TS>(fc.kind, fc.p, fz, z.side, u[i], uz[i],
-                                                 sWq[i + n * j]);
-        }
+    for (int f = 0; f < NFD; ++f)
 #pragma unroll
         for (int i = 0; i < n; ++i)
-            sto<TS>(Rf + i * R.is, orr, (TS)(du[i] + sMinv[i + n * L] * acc[i]));
-    }
+            k[f][i] = k[f][i] + fa[F0 + f][i];
 }
 
 // The kernel.  Seven LDS slots per element node, six of them reused in two
@@ -470,8 +589,9 @@ __device__ __forceinline__ void face_phase(const VolFaces<TS> &fc, const View<co
 //   P23b eta-owner eta-derivatives of the tracer fluxes    -> A, B
 //        zeta-owner vertical diffusion of T, S (same phase) -> C, D
 //   P4b xi-owner   dHT, dHS and d eta complete (written out)
-//   P5  (FACES) xi-owner: the conforming face term added to its line
-template <int N, class TS, class TC, int EPI, int LW, bool FACES>
+//   FACES: after P1's barrier the xi-owner, its state line still in registers,
+//        forms its line's face term, which P4a and P4b add
+template <int N, class TS, class TC, int EPI, int LW, int FACES>
 __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_waves_per_eu(Cfg<N, LW>::template wpe<TS, EPI>())))
     volume_kernel(const VolGeom<TS> geo, const KOps<N + 1, TC> ops, const Phys ph,
                   const View<const TS> U, const Epi<TS> epi, const int64_t nbatch)
@@ -482,6 +602,15 @@ __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_wav
     // registers instead, and runs every stage of one batch before the next.
     constexpr bool STEP = EPI != EPI_RHS;
     constexpr bool PREFETCH = !STEP;
+    // With faces FP64 at N = 4 has no registers to prefetch the tracers, which
+    // are first needed after P1: they are loaded with the neighbours' nodes
+    // (prefetched, 37 VGPRs spilled).
+    // With faces the tendencies stream past the L2, which the neighbours' reads
+    // need (N = 3 FP64 coastline 119 -> 115 us, N = 4 225 -> 216 us), except
+    // where a lane's nodes are adjacent and a streaming store would write the
+    // same line n times (246 -> 401 us).
+    constexpr bool NTS = FACES != FACES_NONE;
+    constexpr int NPRE = FACES && sizeof(TC) == 8 && N == 4 ? 3 : 5;
     // FP64 from N = 6 has no registers to load a step's initial state a phase
     // early (SSP-RK3 at N = 8: 555 us early, 544 us at the use)
     constexpr bool LATE = sizeof(TC) == 8 && N >= 6;
@@ -537,7 +666,15 @@ __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_wav
     const int64_t lw = (geo.xcd_remap && G % kXcds == 0)
                            ? (blockIdx.x % kXcds) * (G / kXcds) + blockIdx.x / kXcds
                            : (int64_t)blockIdx.x;
-    int64_t b = lw;
+    int64_t b = lw, bend = nbatch, bstep = G;
+    if (FACES && geo.xcd_remap && G % kXcds == 0) {
+        // neighbours are read too: each XCD sweeps an eighth of the mesh of its
+        // own, so that they come through its L2
+        const int64_t x = blockIdx.x % kXcds;
+        bstep = G / kXcds;
+        b = nbatch * x / kXcds + blockIdx.x / kXcds;
+        bend = nbatch * (x + 1) / kXcds;
+    }
     if (tid < n * n)
         sDc[tid] = Dc[tid]; // first read in P4b, after P1's barrier
     if constexpr (FACES) {
@@ -552,21 +689,25 @@ __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_wav
         }
     }
     Lines<n, TC> nxt;
+    FaceLine<n> fl;
     if (PREFETCH) {
         const int64_t e0 = elem(b);
-        if (b < nbatch && e0 < geo.E)
-            load_lines<n, EPB, PREFETCH, TS, TC>(nxt, U, geo, b, e0, L0);
+        if (b < bend && e0 < geo.E) {
+            load_lines<n, EPB, NPRE, PREFETCH && !FACES, TS, TC>(nxt, U, geo, b, e0, L0);
+            if constexpr (FACES)
+                fl.load(geo.faces.eface, e0, L0);
+        }
     }
 
     int par = 0;
-    for (; b < nbatch; b += G) {
+    for (; b < bend; b += bstep) {
         const int64_t e = elem(b);
         // P1 reads the prefetched lines in place (the next batch's loads
         // overwrite them only after P1's barrier), so the loop carries no
         // register copies that would wait for those loads.  In a step, nxt
         // is the stage state.
         if (STEP)
-            load_lines<n, EPB, PREFETCH, TS, TC>(nxt, U, geo, b, e, L0);
+            load_lines<n, EPB, 5, false, TS, TC>(nxt, U, geo, b, e, L0);
         Lines<n, TC> &cur = nxt;
         TC acc[step_has_acc(EPI) ? 5 : 1][n];
         if constexpr (step_has_acc(EPI)) {
@@ -595,8 +736,16 @@ __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_wav
         TC pHu[n], pHv[n], ht[n], hs[n];
 
         // ---------------- P1: xi-line (j, k) = (L % n, L / n) ----------------
-        if constexpr (STEP)
+        if constexpr (STEP || FACES)
             load_f<n, TS, TC>(nxt, geo, e, L);
+        if constexpr (NPRE == 3) {
+            const uint32_t uo = state_off<EPB>(U, b, e, L);
+#pragma unroll
+            for (int f = 3; f < 5; ++f)
+#pragma unroll
+                for (int i = 0; i < n; ++i)
+                    nxt.q[f][i] = ldo<TS, TC>(U.p + f * U.fs + i * U.is, uo);
+        }
         {
             TC H[n], u[n], v[n], hinv[n];
 #pragma unroll
@@ -660,18 +809,30 @@ __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_wav
             bar[par][le][0][L] = su;
             bar[par][le][1][L] = sv;
         }
-        __syncthreads();
+        TC fa[FACES ? 5 : 1][n];
+        if constexpr (FACES) {
+            constexpr int CH = face_chunk<N, TC>();
+            FaceNodes<n, CH, TC> fn;
+            fn.template load<0>(fl, U, L);
+            __syncthreads();
+            face_fields<n, CH, 0, FACES == FACES_LF>(fn, fl, geo.faces, U, cur.q, L, sWq, sMinv, fa);
+        } else {
+            __syncthreads();
+        }
 
         if (PREFETCH) {
             // Next batch of this workgroup, in flight during the other phases.
-            const int64_t bn = b + G;
+            const int64_t bn = b + bstep;
             const int64_t en = elem(bn);
             // issued at raised wave priority, so that the SIMD's other wave
             // does not interleave its arithmetic with these loads (6 (N + 1)
             // per lane; 1 % on the FP64 and mixed RHS at 128x128x16, N = 4)
             __builtin_amdgcn_s_setprio(2);
-            if (bn < nbatch && en < geo.E)
-                load_lines<n, EPB, PREFETCH, TS, TC>(nxt, U, geo, bn, en, L);
+            if (bn < bend && en < geo.E) {
+                load_lines<n, EPB, NPRE, PREFETCH && !FACES, TS, TC>(nxt, U, geo, bn, en, L);
+                if constexpr (FACES)
+                    fl.load(geo.faces.eface, en, L);
+            }
             __builtin_amdgcn_s_setprio(0);
         }
 
@@ -755,7 +916,14 @@ __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_wav
             if constexpr (STEP)
                 stage_update<n, 0, 2, EPI>(sc, kv, um, cur.q, acc);
             else
-                write_fields<n, 0, 2, TS, TC>(epi.R, state_off<EPB>(U, b, e, L), kv);
+            {
+                if constexpr (FACES)
+                    add_faces<n, 0, 2>(kv, fa);
+                if (NTS && epi.R.is != 1)
+                    write_fields<n, 0, 2, true>(epi.R, state_off<EPB>(U, b, e, L), kv);
+                else
+                    write_fields<n, 0, 2>(epi.R, state_off<EPB>(U, b, e, L), kv);
+            }
             TC u[n], v[n], hi[n];
 #pragma unroll
             for (int i = 0; i < n; ++i) {
@@ -858,14 +1026,14 @@ __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_wav
             if constexpr (STEP)
                 stage_update<n, 2, 3, EPI>(sc, kv, ut, cur.q, acc);
             else
-                write_fields<n, 2, 3, TS, TC>(epi.R, state_off<EPB>(U, b, e, L), kv);
-        }
-        // ---------------- P5 (FACES): the conforming face term ----------------
-        // Not by the lanes that repeat element E - 1 from another wavefront:
-        // their rereads could meet the owner's final values.
-        if constexpr (FACES) {
-            if (b * EPB + le < geo.E)
-                face_phase<n, TS>(geo.faces, U, epi.R, e, L, sWq, sMinv);
+            {
+                if constexpr (FACES)
+                    add_faces<n, 2, 3>(kv, fa);
+                if (NTS && epi.R.is != 1)
+                    write_fields<n, 2, 3, true>(epi.R, state_off<EPB>(U, b, e, L), kv);
+                else
+                    write_fields<n, 2, 3>(epi.R, state_off<EPB>(U, b, e, L), kv);
+            }
         }
         // No barrier here: this phase reads only its own line's slots and the
         // column integrals of this parity; the next P1 (of the next stage or
@@ -881,7 +1049,7 @@ __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_wav
         }
         if constexpr (STEP)
             if (tid < C::NT && b * EPB + le < geo.E)
-                write_fields<n, 0, 5, TS, TC>(epi.R, state_off<EPB>(U, b, e, L0), cur.q);
+                write_fields<n, 0, 5>(epi.R, state_off<EPB>(U, b, e, L0), cur.q);
     }
 }
 
@@ -916,15 +1084,15 @@ inline int num_cus()
     return cus;
 }
 
-template <int N, class TS, class TC, int EPI, int LW, bool FACES>
+template <int N, class TS, class TC, int EPI, int LW, int FACES>
 hipError_t launch_ne(const VolGeom<TS> &geo, const Ops &ops, const Phys &ph, View<const TS> U,
                      const Epi<TS> &epi, hipStream_t s)
 {
     using C = Cfg<N, LW>;
     if (geo.E <= 0)
         return hipSuccess;
-    // blocked states: whole batches per block; the face phase reads unblocked states only
-    if (U.bb && (U.bb % C::EPB != 0 || FACES))
+    // blocked states: whole batches per block
+    if (U.bb && U.bb % C::EPB != 0)
         return hipErrorInvalidValue;
     const int64_t nbatch = (geo.E + C::EPB - 1) / C::EPB;
     auto kern = volume_kernel<N, TS, TC, EPI, LW, FACES>;
@@ -943,7 +1111,7 @@ hipError_t launch_ne(const VolGeom<TS> &geo, const Ops &ops, const Phys &ph, Vie
         // loads overlap the current batch's arithmetic
         const int wpc = (geo.wg_per_cu > 0 && geo.wg_per_cu < per_cu) ? geo.wg_per_cu : per_cu;
         // what a requested shape amounts to, for the autotuner's report
-        g_rhs_per_cu[sizeof(TS) == 8 ? 0 : 1][LW == 128 ? 0 : LW == 256 ? 1 : 2][N][FACES] =
+        g_rhs_per_cu[sizeof(TS) == 8 ? 0 : 1][LW == 128 ? 0 : LW == 256 ? 1 : 2][N][FACES != FACES_NONE] =
             per_cu;
         grid = (int64_t)num_cus() * wpc;
         if (grid > nbatch)
@@ -971,16 +1139,19 @@ hipError_t launch_n(const VolGeom<TS> &geo, const Ops &ops, const Phys &ph, View
                     const Epi<TS> &epi, hipStream_t s)
 {
     if constexpr (N <= 4) // face plans are built for orders 1-4
-        if (epi.mode == EPI_RHS && geo.faces.eface)
-            return launch_ne<N, TS, TC, EPI_RHS, LW, true>(geo, ops, ph, U, epi, s);
+        if (epi.mode == EPI_RHS && geo.faces.eface) {
+            if (geo.faces.kind == DRF_FLUX_UPWIND)
+                return launch_ne<N, TS, TC, EPI_RHS, LW, FACES_UPWIND>(geo, ops, ph, U, epi, s);
+            return launch_ne<N, TS, TC, EPI_RHS, LW, FACES_LF>(geo, ops, ph, U, epi, s);
+        }
     if (epi.mode == EPI_RHS)
-        return launch_ne<N, TS, TC, EPI_RHS, LW, false>(geo, ops, ph, U, epi, s);
+        return launch_ne<N, TS, TC, EPI_RHS, LW, FACES_NONE>(geo, ops, ph, U, epi, s);
     if constexpr (LW == 128) // whole steps
         switch (epi.mode) {
-        case EPI_STAGE: return launch_ne<N, TS, TC, EPI_STAGE, LW, false>(geo, ops, ph, U, epi, s);
-        case EPI_SSP3: return launch_ne<N, TS, TC, EPI_SSP3, LW, false>(geo, ops, ph, U, epi, s);
-        case EPI_RK4: return launch_ne<N, TS, TC, EPI_RK4, LW, false>(geo, ops, ph, U, epi, s);
-        case EPI_LSRK: return launch_ne<N, TS, TC, EPI_LSRK, LW, false>(geo, ops, ph, U, epi, s);
+        case EPI_STAGE: return launch_ne<N, TS, TC, EPI_STAGE, LW, FACES_NONE>(geo, ops, ph, U, epi, s);
+        case EPI_SSP3: return launch_ne<N, TS, TC, EPI_SSP3, LW, FACES_NONE>(geo, ops, ph, U, epi, s);
+        case EPI_RK4: return launch_ne<N, TS, TC, EPI_RK4, LW, FACES_NONE>(geo, ops, ph, U, epi, s);
+        case EPI_LSRK: return launch_ne<N, TS, TC, EPI_LSRK, LW, FACES_NONE>(geo, ops, ph, U, epi, s);
         default: break;
         }
     return hipErrorInvalidValue;
