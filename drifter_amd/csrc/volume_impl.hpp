@@ -164,6 +164,60 @@ __device__ __forceinline__ void sto(TS *ubase, uint32_t off, TS v)
     else
         *(TS *)((char *)ubase + off) = v;
 }
+// The n adjacent nodes of a xi-line (ADJ: the packed and structure-of-arrays
+// layouts), moved in accesses of up to 16 bytes: with one per node every access
+// of a wavefront touches all the cache lines that the n share, and the L1
+// serves them n times over.
+template <class T> struct Chunk {
+    static constexpr int W = 16 / (int)sizeof(T);
+    typedef T V __attribute__((ext_vector_type(W), aligned(sizeof(T))));
+    typedef T V2 __attribute__((ext_vector_type(2), aligned(sizeof(T))));
+};
+template <int n, class TS, class TC>
+__device__ __forceinline__ void ld_run(const TS *ubase, uint32_t off, TC (&v)[n])
+{
+    using C = Chunk<TS>;
+    const char *p = (const char *)ubase + off;
+    constexpr int nw = n / C::W * C::W, n2 = nw + (C::W == 4 && n - nw >= 2 ? 2 : 0);
+#pragma unroll
+    for (int i = 0; i < nw; i += C::W) {
+        const typename C::V c = *(const typename C::V *)(p + i * sizeof(TS));
+#pragma unroll
+        for (int k = 0; k < C::W; ++k)
+            v[i + k] = (TC)c[k];
+    }
+    if constexpr (n2 > nw) {
+        const typename C::V2 c = *(const typename C::V2 *)(p + nw * sizeof(TS));
+        v[nw] = (TC)c[0];
+        v[nw + 1] = (TC)c[1];
+    }
+    if constexpr (n > n2)
+        v[n2] = (TC)(*(const TS *)(p + n2 * sizeof(TS)));
+}
+template <int n, class TS, class TC>
+__device__ __forceinline__ void st_run(TS *ubase, uint32_t off, const TC (&v)[n])
+{
+    using C = Chunk<TS>;
+    char *p = (char *)ubase + off;
+    constexpr int nw = n / C::W * C::W, n2 = nw + (C::W == 4 && n - nw >= 2 ? 2 : 0);
+#pragma unroll
+    for (int i = 0; i < nw; i += C::W) {
+        typename C::V c;
+#pragma unroll
+        for (int k = 0; k < C::W; ++k)
+            c[k] = (TS)v[i + k];
+        *(typename C::V *)(p + i * sizeof(TS)) = c;
+    }
+    if constexpr (n2 > nw) {
+        typename C::V2 c;
+        c[0] = (TS)v[nw];
+        c[1] = (TS)v[nw + 1];
+        *(typename C::V2 *)(p + nw * sizeof(TS)) = c;
+    }
+    if constexpr (n > n2)
+        *(TS *)(p + n2 * sizeof(TS)) = (TS)v[n2];
+}
+
 // Byte offsets of (element, line) pairs.  32-bit arithmetic is exact: the
 // host checks that every offset of the launch fits in 32 bits.
 //
@@ -256,21 +310,33 @@ __device__ __forceinline__ void load_f(Lines<n, TC> &L, const VolGeom<TS> &geo, 
     }
 }
 
+// Fields [F0, F0 + NFD) of the xi-line at offset so into u[0..]
+template <int n, int F0, int NFD, bool ADJ, class TS, class TC, int NU>
+__device__ __forceinline__ void load_fields(const View<const TS> &U, uint32_t so, TC (&u)[NU][n])
+{
+    if constexpr (ADJ) {
+#pragma unroll
+        for (int f = 0; f < NFD; ++f)
+            ld_run<n, TS, TC>(U.p + (F0 + f) * U.fs, so, u[f]);
+    } else {
+#pragma unroll
+        for (int i = 0; i < n; ++i)
+#pragma unroll
+            for (int f = 0; f < NFD; ++f)
+                u[f][i] = ldo<TS, TC>(U.p + (F0 + f) * U.fs + i * U.is, so);
+    }
+}
+
 // All of P1's global loads are issued here, so that P1 itself waits only for
 // them: a load issued inside P1 would make the wave wait for every store of
 // the previous batch as well (gfx9 counts loads and stores in one in-order
 // counter).
-template <int n, int EPB, int NF, bool WITH_F, class TS, class TC>
+template <int n, int EPB, int NF, bool WITH_F, bool ADJ, class TS, class TC>
 __device__ __forceinline__ void load_lines(Lines<n, TC> &L, const View<const TS> &U,
                                            const VolGeom<TS> &geo, int64_t b, int64_t e, int line)
 {
     const uint32_t uo = state_off<EPB>(U, b, e, line);
-#pragma unroll
-    for (int i = 0; i < n; ++i) {
-#pragma unroll
-        for (int f = 0; f < NF; ++f)
-            L.q[f][i] = ldo<TS, TC>(U.p + f * U.fs + i * U.is, uo);
-    }
+    load_fields<n, 0, NF, ADJ>(U, uo, L.q);
     load_h<n, TS, TC>(L, geo, e, line);
     if (WITH_F)
         load_f<n, TS, TC>(L, geo, e, line);
@@ -280,15 +346,19 @@ constexpr int kXcds = 8; // MI355X: 8 XCDs of 32 CUs
 
 // Writes fields [F0, F0 + NFD) of the thread's xi-line.  so: the line's byte
 // offset in the state views (state_off).
-template <int n, int F0, int NFD, bool NT = false, class TS, class TC>
+template <int n, int F0, int NFD, bool ADJ, bool NT, class TS, class TC>
 __device__ __forceinline__ void write_fields(const View<TS> &R, uint32_t so,
                                              const TC (&kv)[NFD][n])
 {
 #pragma unroll
     for (int f = 0; f < NFD; ++f)
+        if constexpr (ADJ) {
+            st_run<n, TS, TC>(R.p + (F0 + f) * R.fs, so, kv[f]);
+        } else {
 #pragma unroll
-        for (int i = 0; i < n; ++i)
-            sto<TS, NT>(R.p + (F0 + f) * R.fs + i * R.is, so, (TS)kv[f][i]);
+            for (int i = 0; i < n; ++i)
+                sto<TS, NT>(R.p + (F0 + f) * R.fs + i * R.is, so, (TS)kv[f][i]);
+        }
 }
 
 // What the schemes read of the thread's xi-line besides the tendency: the
@@ -298,18 +368,6 @@ __device__ __forceinline__ void write_fields(const View<TS> &R, uint32_t so,
 // spilled 48 VGPRs per lane.)
 constexpr bool step_reads_u0(int epi) { return epi != EPI_RHS && epi != EPI_LSRK; }
 constexpr bool step_has_acc(int epi) { return epi == EPI_RK4 || epi == EPI_LSRK; }
-
-// Fields [F0, F0 + NFD) of the xi-line at offset so
-template <int n, int F0, int NFD, class TS, class TC>
-__device__ __forceinline__ void load_fields(const View<const TS> &U, uint32_t so,
-                                            TC (&u)[NFD][n])
-{
-#pragma unroll
-    for (int f = 0; f < NFD; ++f)
-#pragma unroll
-        for (int i = 0; i < n; ++i)
-            u[f][i] = ldo<TS, TC>(U.p + (F0 + f) * U.fs + i * U.is, so);
-}
 
 // The coefficients of one stage (EpiMode), the dt-proportional one formed from
 // the device dt in adaptive steps.
@@ -591,7 +649,7 @@ __device__ __forceinline__ void add_faces(T (&k)[NFD][n], const T (&fa)[5][n])
 //   P4b xi-owner   dHT, dHS and d eta complete (written out)
 //   FACES: after P1's barrier the xi-owner, its state line still in registers,
 //        forms its line's face term, which P4a and P4b add
-template <int N, class TS, class TC, int EPI, int LW, int FACES>
+template <int N, class TS, class TC, int EPI, int LW, int FACES, bool ADJ>
 __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_waves_per_eu(Cfg<N, LW>::template wpe<TS, EPI>())))
     volume_kernel(const VolGeom<TS> geo, const KOps<N + 1, TC> ops, const Phys ph,
                   const View<const TS> U, const Epi<TS> epi, const int64_t nbatch)
@@ -607,9 +665,8 @@ __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_wav
     // (prefetched, 37 VGPRs spilled).
     // With faces the tendencies stream past the L2, which the neighbours' reads
     // need (N = 3 FP64 coastline 119 -> 115 us, N = 4 225 -> 216 us), except
-    // where a lane's nodes are adjacent and a streaming store would write the
-    // same line n times (246 -> 401 us).
-    constexpr bool NTS = FACES != FACES_NONE;
+    // where a lane's nodes are adjacent and accesses share lines (246 -> 401).
+    constexpr bool NTS = FACES != FACES_NONE && !ADJ;
     constexpr int NPRE = FACES && sizeof(TC) == 8 && N == 4 ? 3 : 5;
     // FP64 from N = 6 has no registers to load a step's initial state a phase
     // early (SSP-RK3 at N = 8: 555 us early, 544 us at the use)
@@ -693,7 +750,7 @@ __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_wav
     if (PREFETCH) {
         const int64_t e0 = elem(b);
         if (b < bend && e0 < geo.E) {
-            load_lines<n, EPB, NPRE, PREFETCH && !FACES, TS, TC>(nxt, U, geo, b, e0, L0);
+            load_lines<n, EPB, NPRE, PREFETCH && !FACES, ADJ, TS, TC>(nxt, U, geo, b, e0, L0);
             if constexpr (FACES)
                 fl.load(geo.faces.eface, e0, L0);
         }
@@ -707,7 +764,7 @@ __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_wav
         // register copies that would wait for those loads.  In a step, nxt
         // is the stage state.
         if (STEP)
-            load_lines<n, EPB, 5, false, TS, TC>(nxt, U, geo, b, e, L0);
+            load_lines<n, EPB, 5, false, ADJ, TS, TC>(nxt, U, geo, b, e, L0);
         Lines<n, TC> &cur = nxt;
         TC acc[step_has_acc(EPI) ? 5 : 1][n];
         if constexpr (step_has_acc(EPI)) {
@@ -742,9 +799,13 @@ __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_wav
             const uint32_t uo = state_off<EPB>(U, b, e, L);
 #pragma unroll
             for (int f = 3; f < 5; ++f)
+                if constexpr (ADJ) {
+                    ld_run<n, TS, TC>(U.p + f * U.fs, uo, nxt.q[f]);
+                } else {
 #pragma unroll
-                for (int i = 0; i < n; ++i)
-                    nxt.q[f][i] = ldo<TS, TC>(U.p + f * U.fs + i * U.is, uo);
+                    for (int i = 0; i < n; ++i)
+                        nxt.q[f][i] = ldo<TS, TC>(U.p + f * U.fs + i * U.is, uo);
+                }
         }
         {
             TC H[n], u[n], v[n], hinv[n];
@@ -829,7 +890,7 @@ __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_wav
             // per lane; 1 % on the FP64 and mixed RHS at 128x128x16, N = 4)
             __builtin_amdgcn_s_setprio(2);
             if (bn < bend && en < geo.E) {
-                load_lines<n, EPB, NPRE, PREFETCH && !FACES, TS, TC>(nxt, U, geo, bn, en, L);
+                load_lines<n, EPB, NPRE, PREFETCH && !FACES, ADJ, TS, TC>(nxt, U, geo, bn, en, L);
                 if constexpr (FACES)
                     fl.load(geo.faces.eface, en, L);
             }
@@ -880,7 +941,7 @@ __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_wav
         // ---------------- P3a: zeta-line (i, j) = L, momentum ----------------
         TC um[2][n]; // initial Hu, Hv for P4a
         if constexpr (step_reads_u0(EPI) && !LATE)
-            load_fields<n, 0, 2>(U, state_off<EPB>(U, b, e, L), um);
+            load_fields<n, 0, 2, ADJ>(U, state_off<EPB>(U, b, e, L), um);
         {
             TC u[n], v[n], hi[n];
 #pragma unroll
@@ -912,17 +973,14 @@ __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_wav
                 kv[1][i] = pHv[i] + sx[S_B * P::SS + i];
             }
             if constexpr (step_reads_u0(EPI) && LATE)
-                load_fields<n, 0, 2>(U, state_off<EPB>(U, b, e, L), um);
+                load_fields<n, 0, 2, ADJ>(U, state_off<EPB>(U, b, e, L), um);
             if constexpr (STEP)
                 stage_update<n, 0, 2, EPI>(sc, kv, um, cur.q, acc);
             else
             {
                 if constexpr (FACES)
                     add_faces<n, 0, 2>(kv, fa);
-                if (NTS && epi.R.is != 1)
-                    write_fields<n, 0, 2, true>(epi.R, state_off<EPB>(U, b, e, L), kv);
-                else
-                    write_fields<n, 0, 2>(epi.R, state_off<EPB>(U, b, e, L), kv);
+                write_fields<n, 0, 2, ADJ, NTS>(epi.R, state_off<EPB>(U, b, e, L), kv);
             }
             TC u[n], v[n], hi[n];
 #pragma unroll
@@ -963,7 +1021,7 @@ __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_wav
         // threads touch the same node of the same slot.
         TC ut[3][n]; // initial eta, HT, HS for P4b
         if constexpr (step_reads_u0(EPI) && !LATE)
-            load_fields<n, 2, 3>(U, state_off<EPB>(U, b, e, L), ut);
+            load_fields<n, 2, 3, ADJ>(U, state_off<EPB>(U, b, e, L), ut);
         {
             TC ftv[n], fsv[n];
 #pragma unroll
@@ -1022,17 +1080,14 @@ __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_wav
                 kv[2][i] = (pHS[i] + sx[S_B * P::SS + i]) + sx[S_D * P::SS + i];
             }
             if constexpr (step_reads_u0(EPI) && LATE)
-                load_fields<n, 2, 3>(U, state_off<EPB>(U, b, e, L), ut);
+                load_fields<n, 2, 3, ADJ>(U, state_off<EPB>(U, b, e, L), ut);
             if constexpr (STEP)
                 stage_update<n, 2, 3, EPI>(sc, kv, ut, cur.q, acc);
             else
             {
                 if constexpr (FACES)
                     add_faces<n, 2, 3>(kv, fa);
-                if (NTS && epi.R.is != 1)
-                    write_fields<n, 2, 3, true>(epi.R, state_off<EPB>(U, b, e, L), kv);
-                else
-                    write_fields<n, 2, 3>(epi.R, state_off<EPB>(U, b, e, L), kv);
+                write_fields<n, 2, 3, ADJ, NTS>(epi.R, state_off<EPB>(U, b, e, L), kv);
             }
         }
         // No barrier here: this phase reads only its own line's slots and the
@@ -1049,7 +1104,7 @@ __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_wav
         }
         if constexpr (STEP)
             if (tid < C::NT && b * EPB + le < geo.E)
-                write_fields<n, 0, 5>(epi.R, state_off<EPB>(U, b, e, L0), cur.q);
+                write_fields<n, 0, 5, ADJ, false>(epi.R, state_off<EPB>(U, b, e, L0), cur.q);
     }
 }
 
@@ -1084,7 +1139,7 @@ inline int num_cus()
     return cus;
 }
 
-template <int N, class TS, class TC, int EPI, int LW, int FACES>
+template <int N, class TS, class TC, int EPI, int LW, int FACES, bool ADJ>
 hipError_t launch_ne(const VolGeom<TS> &geo, const Ops &ops, const Phys &ph, View<const TS> U,
                      const Epi<TS> &epi, hipStream_t s)
 {
@@ -1095,7 +1150,7 @@ hipError_t launch_ne(const VolGeom<TS> &geo, const Ops &ops, const Phys &ph, Vie
     if (U.bb && U.bb % C::EPB != 0)
         return hipErrorInvalidValue;
     const int64_t nbatch = (geo.E + C::EPB - 1) / C::EPB;
-    auto kern = volume_kernel<N, TS, TC, EPI, LW, FACES>;
+    auto kern = volume_kernel<N, TS, TC, EPI, LW, FACES, ADJ>;
     // resident workgroups per CU (queried once per instantiation: the launch
     // path stays free of runtime queries)
     static const int per_cu = [&] {
@@ -1134,6 +1189,15 @@ hipError_t launch_ne(const VolGeom<TS> &geo, const Ops &ops, const Phys &ph, Vie
     return hipGetLastError();
 }
 
+template <int N, class TS, class TC, int EPI, int LW, int FACES>
+hipError_t launch_nl(const VolGeom<TS> &geo, const Ops &ops, const Phys &ph, View<const TS> U,
+                     const Epi<TS> &epi, hipStream_t s)
+{
+    if (U.is == 1)
+        return launch_ne<N, TS, TC, EPI, LW, FACES, true>(geo, ops, ph, U, epi, s);
+    return launch_ne<N, TS, TC, EPI, LW, FACES, false>(geo, ops, ph, U, epi, s);
+}
+
 template <int N, class TS, class TC, int LW>
 hipError_t launch_n(const VolGeom<TS> &geo, const Ops &ops, const Phys &ph, View<const TS> U,
                     const Epi<TS> &epi, hipStream_t s)
@@ -1141,17 +1205,17 @@ hipError_t launch_n(const VolGeom<TS> &geo, const Ops &ops, const Phys &ph, View
     if constexpr (N <= 4) // face plans are built for orders 1-4
         if (epi.mode == EPI_RHS && geo.faces.eface) {
             if (geo.faces.kind == DRF_FLUX_UPWIND)
-                return launch_ne<N, TS, TC, EPI_RHS, LW, FACES_UPWIND>(geo, ops, ph, U, epi, s);
-            return launch_ne<N, TS, TC, EPI_RHS, LW, FACES_LF>(geo, ops, ph, U, epi, s);
+                return launch_nl<N, TS, TC, EPI_RHS, LW, FACES_UPWIND>(geo, ops, ph, U, epi, s);
+            return launch_nl<N, TS, TC, EPI_RHS, LW, FACES_LF>(geo, ops, ph, U, epi, s);
         }
     if (epi.mode == EPI_RHS)
-        return launch_ne<N, TS, TC, EPI_RHS, LW, FACES_NONE>(geo, ops, ph, U, epi, s);
+        return launch_nl<N, TS, TC, EPI_RHS, LW, FACES_NONE>(geo, ops, ph, U, epi, s);
     if constexpr (LW == 128) // whole steps
         switch (epi.mode) {
-        case EPI_STAGE: return launch_ne<N, TS, TC, EPI_STAGE, LW, FACES_NONE>(geo, ops, ph, U, epi, s);
-        case EPI_SSP3: return launch_ne<N, TS, TC, EPI_SSP3, LW, FACES_NONE>(geo, ops, ph, U, epi, s);
-        case EPI_RK4: return launch_ne<N, TS, TC, EPI_RK4, LW, FACES_NONE>(geo, ops, ph, U, epi, s);
-        case EPI_LSRK: return launch_ne<N, TS, TC, EPI_LSRK, LW, FACES_NONE>(geo, ops, ph, U, epi, s);
+        case EPI_STAGE: return launch_nl<N, TS, TC, EPI_STAGE, LW, FACES_NONE>(geo, ops, ph, U, epi, s);
+        case EPI_SSP3: return launch_nl<N, TS, TC, EPI_SSP3, LW, FACES_NONE>(geo, ops, ph, U, epi, s);
+        case EPI_RK4: return launch_nl<N, TS, TC, EPI_RK4, LW, FACES_NONE>(geo, ops, ph, U, epi, s);
+        case EPI_LSRK: return launch_nl<N, TS, TC, EPI_LSRK, LW, FACES_NONE>(geo, ops, ph, U, epi, s);
         default: break;
         }
     return hipErrorInvalidValue;
