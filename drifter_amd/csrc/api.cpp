@@ -397,7 +397,7 @@ drf_status wave_speed(drf_ctx *c, const void *U, int layout, double *out, hipStr
 {
     DRF_REQUIRE(c->precision == DRF_PREC_FP64, DRF_ERR_UNSUPPORTED,
                 "wave speed on the FP64 state only");
-    const int64_t npart = std::min<int64_t>(2048, (c->E + 3) / 4);
+    const int64_t npart = wave_speed_parts(c->order, c->E);
     drf_status st = ensure_red(c, npart + 1);
     if (st)
         return st;
@@ -421,16 +421,15 @@ drf_status adaptive_step(drf_ctx *c, int scheme, double cfl, double dx_min, doub
                          double dt_max, void *U, int layout, double *dt_dev, double *t_dev,
                          hipStream_t s)
 {
-    const int64_t npart = std::min<int64_t>(2048, (c->E + 3) / 4);
+    const int64_t npart = wave_speed_parts(c->order, c->E);
     drf_status st = ensure_red(c, npart + 1);
     if (st)
         return st;
     hipError_t e = launch_wave_speed(c->order, c->E, cview<double>(U, layout, c),
                                      coef_view<double>(c->d_h, c), c->d_red + 1, npart, s);
     if (e == hipSuccess)
-        e = launch_max_reduce(c->d_red + 1, npart, c->d_red, s);
-    if (e == hipSuccess)
-        e = launch_adaptive_dt(c->d_red, dx_min, cfl, dt_min, dt_max, dt_dev, t_dev, s);
+        e = launch_adaptive_dt(c->d_red + 1, npart, c->d_red, dx_min, cfl, dt_min, dt_max, dt_dev,
+                               t_dev, s);
     if (e != hipSuccess)
         return fail(DRF_ERR_HIP, std::string("adaptive dt: ") + hipGetErrorString(e));
     return rk_fused(c, scheme, 0.0, U, layout, s, dt_dev);
@@ -1043,7 +1042,7 @@ drf_status drf_graph_rk_adaptive(drf_ctx *c, int scheme, double cfl, double dx_m
         return st;
     DRF_REQUIRE(n_steps >= 1 && n_steps <= 100000, DRF_ERR_ARG, "n_steps must be 1..100000");
     // the reduction buffer is the context's: size it before capturing
-    st = ensure_red(c, std::min<int64_t>(2048, (c->E + 3) / 4) + 1);
+    st = ensure_red(c, wave_speed_parts(c->order, c->E) + 1);
     if (st)
         return st;
     return capture_graph(c, 0, n_steps, out, [&](hipStream_t cs) {

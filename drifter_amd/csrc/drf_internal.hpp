@@ -240,16 +240,26 @@ inline hipError_t launch_volume_fp32(int order, const VolGeom<float> &geo, const
 }
 
 // Vector kernels (stepper.hip)
+// Workgroups (partial maxima) of the wave-speed reduction: at most 2048, each
+// with the same number of batches of 256 / (N + 1)^2 elements but the last
+// (2048 workgroups on 3,277 batches ran 2 rounds for 1.6 rounds' work).
+inline int64_t wave_speed_parts(int order, int64_t E)
+{
+    const int64_t epb = 256 / ((order + 1) * (order + 1)), nb = (E + epb - 1) / epb;
+    const int64_t rounds = (nb + 2047) / 2048;
+    return (nb + rounds - 1) / rounds;
+}
 hipError_t launch_wave_speed(int order, int64_t E, View<const double> U, View<const double> h,
                              double *partial, int64_t npart, hipStream_t s);
 hipError_t launch_wave_speed_derived(int order, int64_t E, const double *H, const double *u,
                                      const double *v, int64_t es, double *partial,
                                      int64_t npart, hipStream_t s);
 hipError_t launch_max_reduce(const double *partial, int64_t npart, double *out, hipStream_t s);
-// AdaptiveTimeController::compute_dt of the device maximum *cmax into *dt,
+// the same, with AdaptiveTimeController::compute_dt of that maximum into *dt,
 // and *t += dt when t is not null
-hipError_t launch_adaptive_dt(const double *cmax, double dx_min, double cfl, double dt_min,
-                              double dt_max, double *dt, double *t, hipStream_t s);
+hipError_t launch_adaptive_dt(const double *partial, int64_t npart, double *out, double dx_min,
+                              double cfl, double dt_min, double dt_max, double *dt, double *t,
+                              hipStream_t s);
 
 // Face term of an attached face plan (faces_api.cpp): dU += the plan's
 // conforming and mortar contributions.

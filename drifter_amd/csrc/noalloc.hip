@@ -72,7 +72,7 @@ extern "C" drf_status drf_max_wave_speed_noalloc_dev(drf_ctx *c, const void *U, 
         return fail(DRF_ERR_UNSUPPORTED,
                     "drf_max_wave_speed_noalloc_dev: wave speed on the FP64 state only");
     // the same partial count as drf_max_wave_speed_dev, so the two agree bit for bit
-    const int64_t npart = std::min<int64_t>(2048, (c->E + 3) / 4);
+    const int64_t npart = wave_speed_parts(c->order, c->E);
     if (npart > kScratchPartials)
         return fail(DRF_ERR_ARG, "drf_max_wave_speed_noalloc_dev: " + std::to_string(npart) +
                                      " partial maxima exceed the scratch array's " +

@@ -87,3 +87,27 @@ def test_step_is_the_composed_scheme(order, prec, scheme):
         tol = 8 * eps * float(U.abs().max()) + dt * (1e-12 if eps < 1e-12 else 1e-4) * rate
         assert float((got - want).abs().max()) <= tol
         s.close()
+
+
+@pytest.mark.parametrize("order,E", [(1, 64 * 3 + 1), (2, 27), (3, 16 * 2049 + 3), (4, 10 * 2048),
+                                     (6, 11), (8, 3 * 2048 + 1)])
+@pytest.mark.parametrize("layout", [_lib.LAYOUT_SOA, _lib.LAYOUT_LINES])
+def test_wave_speed_at_batch_edges(order, E, layout):
+    """The maximum sits in the last element's last node: every batch of every
+    workgroup (one or two rounds) counts.  max and sqrt are exact."""
+    import torch
+
+    n, nd = order + 1, (order + 1) ** 3
+    print(f"[wave] order={order} E={E} layout={layout}", flush=True)
+    s = PrimitiveEquationsSolver(order)
+    s.initialize(E, np.full(E * nd, 50.0), coriolis=CoriolisParameter(1e-4, 0.0, 0.0))
+    P = torch.zeros((E, 5, n * n, n), dtype=torch.float64, device="cuda")
+    P[:, 0] = 3.0
+    P[-1, 1, -1, -1] = -250.0
+    perm = (1, 0, 2, 3) if layout == _lib.LAYOUT_SOA else (1, 3, 0, 2)
+    U = P.permute(*perm).contiguous().view(-1)
+    assert s.max_wave_speed_dev(U, layout) == float(np.sqrt(9.81 * 50.0) + 250.0 * (1.0 / 50.0))
+    out = torch.zeros(1, dtype=torch.float64, device="cuda")
+    s.max_wave_speed_noalloc_dev(U, out, layout)
+    assert float(out[0]) == s.max_wave_speed_dev(U, layout)
+    s.close()
