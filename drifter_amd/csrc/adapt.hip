@@ -5,12 +5,11 @@
 // compute_directional_mask (src/amr/refinement.cpp:44-161) and the marking
 // loop of AdaptiveMeshRefinement::mark_elements (:488-520, can_refine /
 // can_coarsen :598-606).  A wavefront takes 64 / P elements at a time (P =
-// n^2 rounded up to a power of two, at most 64): their nodes are staged in
-// the wave's slice of LDS with coalesced loads, and each lane owns grid lines
-// of one element, so line variations along xi, eta and zeta read LDS and the
-// per-element reductions stay within a group of P lanes.  Every value is a
-// max, min, difference or single product, so results are bit-identical to
-// the sequential reference loop.
+// n^2 rounded up to a power of two, at most 64): each lane loads xi-lines of
+// one element into registers and stages them in the wave's slice of LDS, where
+// the lanes read eta- and zeta-lines; the per-element reductions stay within a
+// group of P lanes.  Every value is a max, min, difference or single product,
+// so results are bit-identical to the sequential reference loop.
 #include "adapt.hpp"
 #include "drf_internal.hpp"
 
@@ -46,17 +45,42 @@ __host__ __device__ constexpr LineMap line_map(int n)
     return LineMap{P, 64 / P, (n2 + P - 1) / P};
 }
 
-__device__ __forceinline__ double group_max(double v, int P)
+// The value of lane l + O of the 16-lane row (rotated), without the LDS
+template <int O> __device__ __forceinline__ double row_left(double v)
 {
-    for (int o = P >> 1; o > 0; o >>= 1)
-        v = dmax(v, __shfl_xor(v, o));
+    constexpr int ror = 0x120 | (16 - O); // DPP row rotate right
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), ror, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), ror, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+
+// Maximum (minimum) over a group of P lanes, valid in its first lane, which
+// combines the lanes in the order of an xor butterfly.  Steps within 16 lanes
+// rotate in the VALU: through the LDS the five reductions of an element took
+// as long as its line reads.
+template <int P, int O, class F> __device__ __forceinline__ double group_fold(double v, F f)
+{
+    if constexpr (O >= 16)
+        v = f(v, __shfl_xor(v, O));
+    else
+        v = f(v, row_left<O>(v));
+    if constexpr (O > 1)
+        return group_fold<P, O / 2>(v, f);
     return v;
 }
-__device__ __forceinline__ double group_min(double v, int P)
+template <int P> __device__ __forceinline__ double group_max(double v)
 {
-    for (int o = P >> 1; o > 0; o >>= 1)
-        v = dmin(v, __shfl_xor(v, o));
-    return v;
+    if constexpr (P == 1)
+        return v;
+    else
+        return group_fold<P, P / 2>(v, [](double a, double b) { return dmax(a, b); });
+}
+template <int P> __device__ __forceinline__ double group_min(double v)
+{
+    if constexpr (P == 1)
+        return v;
+    else
+        return group_fold<P, P / 2>(v, [](double a, double b) { return dmin(a, b); });
 }
 
 __device__ __forceinline__ void wave_sync_lds()
@@ -66,136 +90,143 @@ __device__ __forceinline__ void wave_sync_lds()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// A wave's elements e0 .. e0 + epw - 1 (cnt of them), nodal values in
-// registers: lane l holds values l, l + 64, ... of the wave's slice.  The
-// kernels load the next elements this way while they work on the current
-// ones, then store them to the slice.  Per-element scalars (h_char, the
-// feature scale) are loaded with them: a load issued after the prefetch
-// would make the wave wait for the prefetch too (gfx9 counts vector-memory
-// loads in one in-order counter).
-template <int n> struct Slice {
-    static constexpr int nd = n * n * n;
-    static constexpr int VPL = (line_map(n).epw * nd + 63) / 64;
-    double v[VPL];
-    __device__ __forceinline__ void load(const double *__restrict__ f, int64_t es, int64_t e0,
-                                         int cnt, int lane)
+// Place of node (i, j, k) in an element's slice of LDS.  The LDS serves 16
+// doubles a clock; at n = 4 the 16 lines of an element, along any axis, met in
+// four banks each, so there the node's two low digits are crossed with k
+// (i ^ k and j ^ k are distinct over every line family).
+template <int n> __device__ __forceinline__ int place(int i, int j, int k)
+{
+    if constexpr (n == 4)
+        return (i ^ k) + 4 * (j ^ k) + 16 * k;
+    return i + n * (j + n * k);
+}
+
+// The xi-lines of a lane (lines gl, gl + P, ... of its element), n adjacent
+// values each, in registers: the kernels load the next elements' lines while
+// they work on the current ones.  Per-element scalars (h_char, the feature
+// scale) are loaded with them: a load issued after the prefetch would make the
+// wave wait for the prefetch too (gfx9 counts vector-memory loads in one
+// in-order counter).
+typedef double pair_t __attribute__((ext_vector_type(2), aligned(8)));
+template <int n> struct Lines1 {
+    static constexpr int P = line_map(n).P, lpl = line_map(n).lpl;
+    double v[lpl][n];
+    __device__ __forceinline__ void load(const double *__restrict__ u, int gl)
     {
 #pragma unroll
-        for (int k = 0; k < VPL; ++k) {
-            const int idx = lane + 64 * k;
-            if (idx < cnt * nd) {
-                const int el = idx / nd, d = idx - el * nd;
-                v[k] = f[(e0 + el) * es + d];
+        for (int t = 0; t < lpl; ++t) {
+            const int L = gl + t * P;
+            if (L < n * n) {
+#pragma unroll
+                for (int i = 0; i + 1 < n; i += 2) {
+                    const pair_t c = *(const pair_t *)(u + L * n + i);
+                    v[t][i] = c[0];
+                    v[t][i + 1] = c[1];
+                }
+                if constexpr (n & 1)
+                    v[t][n - 1] = u[L * n + n - 1];
             }
-        }
-    }
-    __device__ __forceinline__ void store(double *u, int cnt, int lane) const
-    {
-#pragma unroll
-        for (int k = 0; k < VPL; ++k) {
-            const int idx = lane + 64 * k;
-            if (idx < cnt * nd)
-                u[idx] = v[k];
         }
     }
 };
 
 // Pass 1: raw indicator value[e] = (max - min) * h_char[e] and the
-// directional mask; partial[block] = max of the block's values.
+// directional mask; partial[block] = max of the block's values.  HBM-bound
+// (nd 8 + 17 B per element) once the LDS is out of the way: 196,400 elements,
+// N = 3 40.5 us with conflicting line reads and reductions through the LDS,
+// now 25.0 us.
 template <int n>
 __global__ void __launch_bounds__(64 * kWaves)
     estimate_kernel(int64_t E, const double *__restrict__ field, int64_t es,
                     const double *__restrict__ hchar, double smooth, double *__restrict__ value,
                     uint8_t *__restrict__ mask, double *__restrict__ partial)
 {
-    extern __shared__ double sm[];
+    constexpr int n2 = n * n, nd = n2 * n;
+    constexpr LineMap lm = line_map(n);
+    __shared__ double sm[kWaves * lm.epw * nd];
     __shared__ double red[kWaves];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int n2 = n * n, nd = n2 * n;
-    const LineMap lm = line_map(n);
     const int g = lane / lm.P, gl = lane % lm.P; // element within the wave, lane within it
-    double *u = sm + (size_t)w * lm.epw * nd;
+    double *ue = sm + (w * lm.epw + g) * nd;
     double bmax = 0.0;
-    const int64_t waves = (int64_t)gridDim.x * kWaves;
-    const int64_t step = waves * lm.epw;
-    auto count = [&](int64_t e) { return (E - e < lm.epw) ? (int)(E - e) : lm.epw; };
-    Slice<n> nx;
-    int64_t e0 = ((int64_t)blockIdx.x * kWaves + w) * lm.epw;
-    double hc_next = 0.0; // h_char of the lane's element in the next slice
-    auto load_next = [&](int64_t e) {
-        nx.load(field, es, e, count(e), lane);
-        hc_next = (g < count(e)) ? hchar[e + g] : 0.0;
+    const int64_t step = (int64_t)gridDim.x * kWaves * lm.epw;
+    Lines1<n> nx;
+    int64_t e = ((int64_t)blockIdx.x * kWaves + w) * lm.epw + g; // the lane's element
+    double hc_next = 0.0;
+    auto load_next = [&](int64_t en) {
+        if (en < E) {
+            nx.load(field + en * es, gl);
+            hc_next = hchar[en];
+        }
     };
-    if (e0 < E)
-        load_next(e0);
-    for (; e0 < E; e0 += step) {
-        const int cnt = count(e0);
-        nx.store(u, cnt, lane);
+    load_next(e);
+    for (int64_t e0 = e - g; e0 < E; e0 += step, e += step) {
+        const bool on = e < E;
         const double hc = hc_next;
-        if (e0 + step < E)
-            load_next(e0 + step);
-        wave_sync_lds();
         double hi = -INFINITY, lo = INFINITY, vx = 0.0, vy = 0.0, vz = 0.0;
-        if (g < cnt) {
-            const double *ue = u + g * nd;
+        if (on) {
+            // xi-line (j, k) = (a, b): also the element's max and min
+#pragma unroll
             for (int t = 0; t < lm.lpl; ++t) {
-                const int L = gl + t * lm.P;
-                if (L >= n2)
-                    break;
-                const int a = L % n, b = L / n;
-                // xi-line (j, k) = (a, b): also the element's max and min
-                double l0 = ue[b * n2 + a * n], h0 = l0;
-                for (int i = 1; i < n; ++i) {
-                    const double v = ue[b * n2 + a * n + i];
-                    l0 = dmin(l0, v);
-                    h0 = dmax(h0, v);
+                const int L = gl + t * lm.P, a = L % n, b = L / n;
+                if (L < n2) {
+                    double l0 = nx.v[t][0], h0 = l0;
+#pragma unroll
+                    for (int i = 0; i < n; ++i) {
+                        const double v = nx.v[t][i];
+                        ue[place<n>(i, a, b)] = v;
+                        l0 = dmin(l0, v);
+                        h0 = dmax(h0, v);
+                    }
+                    vx = dmax(vx, h0 - l0);
+                    hi = dmax(hi, h0);
+                    lo = dmin(lo, l0);
                 }
-                vx = dmax(vx, h0 - l0);
-                hi = dmax(hi, h0);
-                lo = dmin(lo, l0);
-                // eta-line (i, k) = (a, b)
-                l0 = ue[b * n2 + a];
-                h0 = l0;
-                for (int j = 1; j < n; ++j) {
-                    const double v = ue[b * n2 + j * n + a];
-                    l0 = dmin(l0, v);
-                    h0 = dmax(h0, v);
-                }
-                vy = dmax(vy, h0 - l0);
-                // zeta-line (i, j) = (a, b)
-                l0 = ue[b * n + a];
-                h0 = l0;
-                for (int k = 1; k < n; ++k) {
-                    const double v = ue[k * n2 + b * n + a];
-                    l0 = dmin(l0, v);
-                    h0 = dmax(h0, v);
-                }
-                vz = dmax(vz, h0 - l0);
             }
         }
-        hi = group_max(hi, lm.P);
-        lo = group_min(lo, lm.P);
-        vx = group_max(vx, lm.P);
-        vy = group_max(vy, lm.P);
-        vz = group_max(vz, lm.P);
-        if (g < cnt) {
-            const int64_t e = e0 + g;
+        load_next(e + step);
+        wave_sync_lds();
+        if (on) {
+#pragma unroll
+            for (int t = 0; t < lm.lpl; ++t) {
+                const int L = gl + t * lm.P, a = L % n, b = L / n;
+                if (L < n2) {
+                    // eta-line (i, k) = (a, b), zeta-line (i, j) = (a, b)
+                    double l0 = ue[place<n>(a, 0, b)], h0 = l0;
+                    double l1 = ue[place<n>(a, b, 0)], h1 = l1;
+#pragma unroll
+                    for (int j = 1; j < n; ++j) {
+                        const double v = ue[place<n>(a, j, b)], q = ue[place<n>(a, b, j)];
+                        l0 = dmin(l0, v);
+                        h0 = dmax(h0, v);
+                        l1 = dmin(l1, q);
+                        h1 = dmax(h1, q);
+                    }
+                    vy = dmax(vy, h0 - l0);
+                    vz = dmax(vz, h1 - l1);
+                }
+            }
+        }
+        hi = group_max<lm.P>(hi);
+        lo = group_min<lm.P>(lo);
+        vx = group_max<lm.P>(vx);
+        vy = group_max<lm.P>(vy);
+        vz = group_max<lm.P>(vz);
+        if (on && gl == 0) {
             const double val = (hi - lo) * hc;
             bmax = dmax(bmax, val);
-            if (gl == 0) {
-                const double mv = dmax(dmax(vx, vy), vz);
-                uint8_t m = 0;
-                if (!(mv < 1e-14)) {
-                    const double thr = smooth * mv;
-                    m = (vx > thr ? 1 : 0) | (vy > thr ? 2 : 0) | (vz > thr ? 4 : 0);
-                }
-                value[e] = val;
-                mask[e] = m;
+            const double mv = dmax(dmax(vx, vy), vz);
+            uint8_t m = 0;
+            if (!(mv < 1e-14)) {
+                const double thr = smooth * mv;
+                m = (vx > thr ? 1 : 0) | (vy > thr ? 2 : 0) | (vz > thr ? 4 : 0);
             }
+            value[e] = val;
+            mask[e] = m;
         }
-        wave_sync_lds(); // the slice is reloaded for the next elements
+        wave_sync_lds(); // the slice is rewritten for the next elements
     }
-    bmax = group_max(bmax, 64);
+    bmax = group_max<64>(bmax);
     if (lane == 0)
         red[w] = bmax;
     __syncthreads();
@@ -206,7 +237,6 @@ __global__ void __launch_bounds__(64 * kWaves)
         partial[blockIdx.x] = m;
     }
 }
-
 
 // Pass 2: global max from the partials (every block), normalisation,
 // thresholds, then mark_elements when levels are given.
@@ -269,76 +299,90 @@ __device__ __forceinline__ uint16_t to_bf16(float f)
 }
 
 // Nodal -> modal by sum factorisation, line-parallel: three passes of n x n
-// contractions (xi, then eta, then zeta) through the wave's LDS slice, lanes
-// owning grid lines.  OUT = double (coefficients) or uint16_t (BF16
-// features, scaled, mean mode zeroed).
+// contractions, xi from the lane's own line in registers, then eta and zeta
+// through the wave's LDS slice, lanes owning grid lines.  OUT = double
+// (coefficients) or uint16_t (BF16 features, scaled, mean mode zeroed).
+// 39,280 elements, N = 3, BF16: 9.1 us with all three passes through
+// conflicting LDS slices, now 7.0 us.
 template <int n, class OUT>
 __global__ void __launch_bounds__(64 * kWaves)
     modal_kernel(int64_t E, const double *__restrict__ u, int64_t es, ModalOps ops,
                  OUT *__restrict__ out, int64_t out_stride, int out_offset, double scale,
                  const double *__restrict__ elem_scale)
 {
-    extern __shared__ double sm[];
+    constexpr int n2 = n * n, nd = n2 * n;
+    constexpr LineMap lm = line_map(n);
+    __shared__ double sm[kWaves * lm.epw * nd];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int n2 = n * n, nd = n2 * n;
-    const LineMap lm = line_map(n);
     const int g = lane / lm.P, gl = lane % lm.P;
-    double *a = sm + (size_t)w * 2 * lm.epw * nd, *bb = a + lm.epw * nd;
-    const int64_t waves = (int64_t)gridDim.x * kWaves;
-    const int64_t step = waves * lm.epw;
-    auto count = [&](int64_t e) { return (E - e < lm.epw) ? (int)(E - e) : lm.epw; };
-    Slice<n> nx;
-    int64_t e0 = ((int64_t)blockIdx.x * kWaves + w) * lm.epw;
+    double *ue = sm + (w * lm.epw + g) * nd;
+    const int64_t step = (int64_t)gridDim.x * kWaves * lm.epw;
+    Lines1<n> nx;
+    int64_t e = ((int64_t)blockIdx.x * kWaves + w) * lm.epw + g;
     double es_next = 1.0; // elem_scale of the lane's element in the next slice
-    auto load_next = [&](int64_t e) {
-        nx.load(u, es, e, count(e), lane);
-        es_next = (elem_scale && g < count(e)) ? elem_scale[e + g] : 1.0;
+    auto load_next = [&](int64_t en) {
+        if (en < E) {
+            nx.load(u + en * es, gl);
+            es_next = elem_scale ? elem_scale[en] : 1.0;
+        }
     };
-    if (e0 < E)
-        load_next(e0);
-    for (; e0 < E; e0 += step) {
-        const int cnt = count(e0);
-        nx.store(a, cnt, lane);
+    load_next(e);
+    for (int64_t e0 = e - g; e0 < E; e0 += step, e += step) {
+        const bool act = e < E;
         const double sc = elem_scale ? scale * es_next : scale; // used after the next load
-        if (e0 + step < E)
-            load_next(e0 + step);
-        wave_sync_lds();
-        const bool act = g < cnt;
-        double *ae = a + g * nd, *be = bb + g * nd;
         if (act) // xi: b[p + n L] = sum_i Vi[p][i] a[i + n L], L = (j, k)
-            for (int L = gl; L < n2; L += lm.P)
-                for (int p = 0; p < n; ++p) {
-                    double s = 0.0;
-                    for (int i = 0; i < n; ++i)
-                        s += ops.Vinv[p * kMaxN + i] * ae[L * n + i];
-                    be[L * n + p] = s;
-                }
+#pragma unroll
+            for (int t = 0; t < lm.lpl; ++t) {
+                const int L = gl + t * lm.P;
+                if (L < n2)
+#pragma unroll
+                    for (int p = 0; p < n; ++p) {
+                        double s = 0.0;
+#pragma unroll
+                        for (int i = 0; i < n; ++i)
+                            s += ops.Vinv[p * kMaxN + i] * nx.v[t][i];
+                        ue[place<n>(p, L % n, L / n)] = s;
+                    }
+            }
+        load_next(e + step);
         wave_sync_lds();
-        if (act) // eta: a[p + n(q + n k)] = sum_j Vi[q][j] b[p + n(j + n k)], L = (p, k)
+        if (act) // eta, in place along the lane's line (p, k)
             for (int L = gl; L < n2; L += lm.P) {
                 const int p = L % n, k = L / n;
+                double x[n];
+#pragma unroll
+                for (int j = 0; j < n; ++j)
+                    x[j] = ue[place<n>(p, j, k)];
+#pragma unroll
                 for (int q = 0; q < n; ++q) {
                     double s = 0.0;
+#pragma unroll
                     for (int j = 0; j < n; ++j)
-                        s += ops.Vinv[q * kMaxN + j] * be[k * n2 + j * n + p];
-                    ae[k * n2 + q * n + p] = s;
+                        s += ops.Vinv[q * kMaxN + j] * x[j];
+                    ue[place<n>(p, q, k)] = s;
                 }
             }
         wave_sync_lds();
         if (act) { // zeta: coef[L + n2 r] = sum_k Vi[r][k] a[L + n2 k], L = (p, q)
-            const int64_t e = e0 + g;
             OUT *dst = out + e * out_stride + out_offset;
-            for (int L = gl; L < n2; L += lm.P)
+            for (int L = gl; L < n2; L += lm.P) {
+                double x[n];
+#pragma unroll
+                for (int k = 0; k < n; ++k)
+                    x[k] = ue[place<n>(L % n, L / n, k)];
+#pragma unroll
                 for (int r = 0; r < n; ++r) {
                     double s = 0.0;
+#pragma unroll
                     for (int k = 0; k < n; ++k)
-                        s += ops.Vinv[r * kMaxN + k] * ae[k * n2 + L];
+                        s += ops.Vinv[r * kMaxN + k] * x[k];
                     const int d = L + n2 * r;
                     if constexpr (sizeof(OUT) == 8)
                         dst[d] = s;
                     else // features: the element mean (mode 0) carries no variation
                         dst[d] = (d == 0) ? (uint16_t)0 : to_bf16((float)(s * sc));
                 }
+            }
         }
         wave_sync_lds();
     }
@@ -361,9 +405,8 @@ hipError_t launch_estimate(int n, int64_t E, const double *field, int64_t es, co
     if (E <= 0)
         return hipSuccess;
     const unsigned g1 = grid_for(n, E, kEstimatorPartials);
-    const size_t lds = sizeof(double) * (size_t)kWaves * line_map(n).epw * n * n * n;
 #define DRF_EST(NN)                                                                           \
-    hipLaunchKernelGGL(estimate_kernel<NN>, dim3(g1), dim3(64 * kWaves), lds, s, E, field, es,  \
+    hipLaunchKernelGGL(estimate_kernel<NN>, dim3(g1), dim3(64 * kWaves), 0, s, E, field, es,  \
                        hchar, p.smoothness_factor, value, mask, partial)
     switch (n) {
     case 2: DRF_EST(2); break;
@@ -394,14 +437,13 @@ hipError_t launch_modal(int n, int64_t E, const double *u, int64_t es, const Mod
     if (E <= 0)
         return hipSuccess;
     const unsigned g = grid_for(n, E, 8192);
-    const size_t lds = sizeof(double) * (size_t)kWaves * 2 * line_map(n).epw * n * n * n;
 #define DRF_MODAL(NN)                                                                         \
     do {                                                                                      \
         if (coef)                                                                             \
-            hipLaunchKernelGGL((modal_kernel<NN, double>), dim3(g), dim3(64 * kWaves), lds, s, E, \
+            hipLaunchKernelGGL((modal_kernel<NN, double>), dim3(g), dim3(64 * kWaves), 0, s, E, \
                                u, es, ops, coef, out_stride, out_offset, scale, elem_scale);  \
         else                                                                                  \
-            hipLaunchKernelGGL((modal_kernel<NN, uint16_t>), dim3(g), dim3(64 * kWaves), lds, s,  \
+            hipLaunchKernelGGL((modal_kernel<NN, uint16_t>), dim3(g), dim3(64 * kWaves), 0, s,  \
                                E, u, es, ops, bf16, out_stride, out_offset, scale, elem_scale); \
     } while (0)
     switch (n) {
