@@ -106,7 +106,8 @@ template <int R, bool TRAIN> struct alignas(16) Smem {
     uint16_t d2[TRAIN ? R : 1][LH], d1[TRAIN ? R : 1][LH];
     float g1[TRAIN ? R : 1][NH], g2[TRAIN ? R : 1][NH];
     float d3[TRAIN ? R : 1];
-    float red[TRAIN ? 4 * NH : 1];
+    float red[TRAIN ? 3 : 1][TRAIN ? 4 * NH : 1];
+    float tail[TRAIN ? 8 : 1];
 };
 
 // Weights to LDS: W1, W2 as BF16 (already rounded in wq), W3 as the float
@@ -115,10 +116,14 @@ template <int R, bool TRAIN>
 __device__ void stage_weights(Smem<R, TRAIN> &s, const float *__restrict__ w,
                               const uint16_t *__restrict__ wq)
 {
-    for (int i = threadIdx.x; i < NH * NI; i += blockDim.x)
-        s.w1[i / NI][i % NI] = wq[i];
-    for (int i = threadIdx.x; i < NH * NH; i += blockDim.x)
-        s.w2[i / NH][i % NH] = wq[NH * NI + i];
+    // 16-byte pieces (rows and pitches are multiples of 16 bytes): value by
+    // value the staging was a third of a minibatch's kernel
+    for (int i = threadIdx.x; i < NH * NI / 8; i += blockDim.x)
+        *reinterpret_cast<uint4 *>(&s.w1[i / (NI / 8)][i % (NI / 8) * 8]) =
+            reinterpret_cast<const uint4 *>(wq)[i];
+    for (int i = threadIdx.x; i < NH * NH / 8; i += blockDim.x)
+        *reinterpret_cast<uint4 *>(&s.w2[i / (NH / 8)][i % (NH / 8) * 8]) =
+            reinterpret_cast<const uint4 *>(wq + NH * NI)[i];
     for (int i = threadIdx.x; i < NH; i += blockDim.x) {
         s.w3[i] = bf2f(wq[NH * NI + NH * NH + i]);
         s.b1[i] = w[OB1 + i];
@@ -228,11 +233,7 @@ __global__ void __launch_bounds__(64 * kInferWaves)
     for (int q = threadIdx.x; q < 4 * 8 * 64; q += 64 * kInferWaves) {
         const int ln = q & 63, ms = q >> 6, mb = ms >> 3, st = ms & 7;
         const uint16_t *src = wq + (16 * mb + (ln & 15)) * NI + 32 * (ln >> 4) + 4 * st;
-        bf16x4 v;
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-            v[t] = (short)src[t];
-        f1[q] = v;
+        f1[q] = *reinterpret_cast<const bf16x4 *>(src);
     }
     for (int q = threadIdx.x; q < NH; q += 64 * kInferWaves) {
         b1s[q] = w[OB1 + q];
@@ -432,68 +433,69 @@ __global__ void __launch_bounds__(256)
             P[OW2 + (m0 + (lane >> 4) * 4 + t) * NH + n0 + (lane & 15)] = gw2[q][t];
     }
     __syncthreads();
-    // per-column sums over the four row groups, in a fixed order
-    float *red = s.red;
-    red[rg * NH + col] = gb1;
-    __syncthreads();
-    if (threadIdx.x < NH)
-        P[OB1 + col] = red[col] + red[NH + col] + red[2 * NH + col] + red[3 * NH + col];
-    __syncthreads();
-    red[rg * NH + col] = gb2;
-    __syncthreads();
-    if (threadIdx.x < NH)
-        P[OB2 + col] = red[col] + red[NH + col] + red[2 * NH + col] + red[3 * NH + col];
-    __syncthreads();
-    red[rg * NH + col] = gw3;
-    __syncthreads();
-    if (threadIdx.x < NH)
-        P[OW3 + col] = red[col] + red[NH + col] + red[2 * NH + col] + red[3 * NH + col];
-    __syncthreads();
-    // b3 and loss: block sums
-    red[threadIdx.x] = gb3;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        float a = 0.f;
-        for (int i = 0; i < 256; ++i)
-            a += red[i];
-        P[OB3] = a;
+    // per-column sums over the four row groups, and the sums of b3's gradient
+    // (held by column 0) and the loss (by the first R lanes), in fixed orders
+    s.red[0][rg * NH + col] = gb1;
+    s.red[1][rg * NH + col] = gb2;
+    s.red[2][rg * NH + col] = gw3;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1)
+        loss += __shfl_xor(loss, o);
+    if (col == 0) {
+        s.tail[rg] = gb3;
+        s.tail[4 + rg] = loss;
     }
     __syncthreads();
-    red[threadIdx.x] = loss;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        float a = 0.f;
-        for (int i = 0; i < 256; ++i)
-            a += red[i];
-        lpart[blockIdx.x] = a;
+    if (threadIdx.x < 3 * NH) {
+        const float *r = s.red[rg];
+        P[(rg == 0 ? OB1 : rg == 1 ? OB2 : OW3) + col] =
+            r[col] + r[NH + col] + r[2 * NH + col] + r[3 * NH + col];
+    }
+    if (threadIdx.x == 3 * NH) {
+        P[OB3] = s.tail[0] + s.tail[1] + s.tail[2] + s.tail[3];
+        lpart[blockIdx.x] = s.tail[4] + s.tail[5] + s.tail[6] + s.tail[7];
     }
 }
 
 // Sum of the partial gradients (fixed order), then either write the
 // gradient or take one Adam step on the master weights and refresh their
-// BF16 copies.
+// BF16 copies.  A workgroup takes 64 parameters, its wavefronts a quarter of
+// the partials each: with one thread for a parameter's whole sum the kernel
+// was that sum's chain of loads on 49 workgroups (64 partials: 4.9 us, now
+// 3.7 us).
 __global__ void __launch_bounds__(256)
     mlp_reduce_kernel(int nparts, const float *__restrict__ partial,
                       const float *__restrict__ lpart, float inv_b, float *__restrict__ grad,
                       float *__restrict__ loss, AdamStep adam, float *__restrict__ w,
                       float *__restrict__ m, float *__restrict__ v, uint16_t *__restrict__ wq)
 {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    // Sums in partial order (deterministic); unrolled so that the loads of
-    // a group are in flight together.
-    if (p == 0 && loss) {
-        float a = 0.f;
-#pragma unroll 16
-        for (int i = 0; i < nparts; ++i)
-            a += lpart[i];
-        *loss = a * inv_b;
-    }
-    if (p >= NP)
-        return;
+    __shared__ float quarter[4][64];
+    const int lane = threadIdx.x & 63, part = threadIdx.x >> 6;
+    const int p = blockIdx.x * 64 + lane;
+    const int per = (nparts + 3) / 4, first = part * per;
+    const int last = first + per < nparts ? first + per : nparts;
     float g = 0.f;
+    if (p < NP) {
 #pragma unroll 16
-    for (int i = 0; i < nparts; ++i)
-        g += partial[(size_t)i * NP + p];
+        for (int i = first; i < last; ++i)
+            g += partial[(size_t)i * NP + p];
+    }
+    quarter[part][lane] = g;
+    // the loss: lane sums of every 64th partial, then the lanes
+    if (blockIdx.x == 0 && part == 1 && loss) {
+        float a = 0.f;
+        for (int i = lane; i < nparts; i += 64)
+            a += lpart[i];
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1)
+            a += __shfl_xor(a, o);
+        if (lane == 0)
+            *loss = a * inv_b;
+    }
+    __syncthreads();
+    if (part != 0 || p >= NP)
+        return;
+    g = quarter[0][lane] + quarter[1][lane] + quarter[2][lane] + quarter[3][lane];
     if (grad)
         grad[p] = g;
     if (adam.lr != 0.f) {
@@ -523,13 +525,17 @@ __global__ void __launch_bounds__(256)
     }
 }
 
-constexpr int kRowsTrain = 32;
+// Rows per tile: 16 while that gives every tile a CU of its own (the kernel is
+// then one tile's chain of phases: 2,048 rows 16.7 us in tiles of 32, 10.9
+// us in tiles of 16), 32 for more (half the partial gradients).
+constexpr int64_t kSmallBatch = 16 * 256;
+int rows_per_tile(int64_t n) { return n <= kSmallBatch ? 16 : 32; }
 
 } // namespace
 
 int mlp_grad_parts(int64_t n)
 {
-    const int64_t tiles = (n + kRowsTrain - 1) / kRowsTrain;
+    const int64_t rows = rows_per_tile(n), tiles = (n + rows - 1) / rows;
     return (int)(tiles < kMlpMaxParts ? tiles : kMlpMaxParts);
 }
 
@@ -567,12 +573,16 @@ hipError_t launch_mlp_grad(int64_t n, const uint16_t *X, const float *y, float *
         return hipSuccess;
     const int parts = mlp_grad_parts(n);
     const float inv_b = 1.0f / (float)n;
-    hipLaunchKernelGGL(mlp_grad_kernel<kRowsTrain>, dim3(parts), dim3(256), 0, s, n, X, y, w, wq,
-                       inv_b, partial, lpart);
+    if (rows_per_tile(n) == 16)
+        hipLaunchKernelGGL(mlp_grad_kernel<16>, dim3(parts), dim3(256), 0, s, n, X, y, w, wq,
+                           inv_b, partial, lpart);
+    else
+        hipLaunchKernelGGL(mlp_grad_kernel<32>, dim3(parts), dim3(256), 0, s, n, X, y, w, wq,
+                           inv_b, partial, lpart);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess)
         return e;
-    hipLaunchKernelGGL(mlp_reduce_kernel, dim3((kMlpParams + 255) / 256), dim3(256), 0, s, parts,
+    hipLaunchKernelGGL(mlp_reduce_kernel, dim3((kMlpParams + 63) / 64), dim3(256), 0, s, parts,
                        partial, lpart, inv_b, grad, loss, adam, w, m, v, wq);
     return hipGetLastError();
 }
