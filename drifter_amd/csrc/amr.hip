@@ -468,12 +468,22 @@ __global__ void __launch_bounds__(kThreads)
     }
 }
 
-template <int64_t PER>
+template <int64_t PER, int64_t CAP = 4096>
 unsigned grid_for(int64_t units)
 {
     const int64_t nb = (units + PER - 1) / PER;
-    return (unsigned)(nb < 4096 ? nb : 4096);
+    return (unsigned)(nb < CAP ? nb : CAP);
 }
+
+// interp_boxes_kernel gets one workgroup per batch: its phases wait on each
+// other, and a workgroup that begins as another ends fills those waits, where a
+// grid-stride loop runs them one after another behind its closing barrier.
+// Six fields, 64 x 64 x 8 elements refined in a band: N = 4 256.8 us with 4096
+// workgroups, 251.1 with one per batch; a narrower band N = 3 113.2 and 111.4,
+// N = 4 241.9 and 239.0, N = 5 to 8 the same; 2048 workgroups are slower
+// (N = 3 128.4, N = 4 253.2).  The cap keeps the launch's threads below 2^32;
+// beyond it the kernel strides.
+constexpr int64_t kBoxGrid = int64_t(1) << 23;
 
 template <int N>
 hipError_t interp_n(BoxMode mode, int mask, int64_t n_out, int64_t n_src, const BoxFields &bf,
@@ -499,8 +509,8 @@ hipError_t interp_n(BoxMode mode, int mask, int64_t n_out, int64_t n_src, const 
                            blk, 0, s, mask, n_src, n_src, U, es, (int64_t)0, idx, ns, out, os);
         break;
     default:
-        hipLaunchKernelGGL((interp_boxes_kernel<N>), dim3(grid_for<S::BPB>(n_out)), blk, 0, s,
-                           n_out, n_src, bf, idx, boxes, ns);
+        hipLaunchKernelGGL((interp_boxes_kernel<N>), dim3(grid_for<S::BPB, kBoxGrid>(n_out)), blk, 0,
+                           s, n_out, n_src, bf, idx, boxes, ns);
         break;
     }
     return hipGetLastError();
