@@ -206,12 +206,16 @@ __device__ void forward_tile(Smem<R, TRAIN> &s, float b3)
 // layers are computed transposed, H^T = W X^T, so a layer's accumulator
 // (lane l: hidden units 16 mb + 4 (l / 16) + t of row l % 16) is exactly the
 // next layer's B operand (K index 4 (l / 16) + t of K-step mb, column l % 16):
-// activations never leave registers.  W2 lives in registers (its 16 A
-// fragments); W1's 32 fragments are read from LDS, laid out per (mb, step,
-// lane) so every read is one conflict-free 8-byte access.  Layer 1's K order
-// is permuted (step s of lane group g contracts inputs 32 g + 4 s .. + 3) so
-// each lane's 32 inputs of a row are contiguous: four 16-byte loads, issued
-// for the next tile before the current one is computed.
+// activations never leave registers.  W1's 32 and W2's 16 fragments are read
+// from LDS, laid out per (mb, step, lane) so every read is one conflict-free
+// 8-byte access.  Layer 1's K order is permuted (step s of lane group g
+// contracts inputs 32 g + 4 s .. + 3) so each lane's 32 inputs of a row are
+// contiguous: four 16-byte loads, issued for the next tile before the current
+// one is computed, and for the first before the weights are staged.
+// Bound by the GELUs and by what hides one tile's chain, the resident waves:
+// with the fragments in registers (194 VGPRs, two waves per SIMD) the two
+// feature passes, this and the decisions took 72.2 us for 196,400 rows and
+// 331.6 us for a million; four waves per SIMD take 68.9 and 323.1 us.
 typedef __bf16 bf16x2v __attribute__((ext_vector_type(2)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 
@@ -223,37 +227,30 @@ __device__ __forceinline__ uint32_t pack_bf16(float a, float b)
 
 constexpr int kInferWaves = 4;
 
-__global__ void __launch_bounds__(64 * kInferWaves)
+__global__ void __launch_bounds__(64 * kInferWaves, 4)
     mlp_infer_kernel(int64_t n, const uint16_t *__restrict__ X, const float *__restrict__ w,
                      const uint16_t *__restrict__ wq, float *__restrict__ pred)
 {
-    // W1 fragments: f1[(mb * 8 + s) * 64 + lane][t] = W1[16 mb + lane % 16][32 (lane / 16) + 4 s + t]
-    __shared__ bf16x4 f1[4 * 8 * 64];
+    // f1[(mb * 8 + s) * 64 + lane][t] = W1[16 mb + lane % 16][32 (lane / 16) + 4 s + t]
+    // f2s[(mb * 4 + s) * 64 + lane][t] = W2[16 mb + lane % 16][16 s + 4 (lane / 16) + t]
+    __shared__ bf16x4 f1[4 * 8 * 64], f2s[4 * 4 * 64];
     __shared__ __align__(16) float b1s[NH], b2s[NH], w3s[NH];
-    for (int q = threadIdx.x; q < 4 * 8 * 64; q += 64 * kInferWaves) {
-        const int ln = q & 63, ms = q >> 6, mb = ms >> 3, st = ms & 7;
-        const uint16_t *src = wq + (16 * mb + (ln & 15)) * NI + 32 * (ln >> 4) + 4 * st;
-        f1[q] = *reinterpret_cast<const bf16x4 *>(src);
-    }
-    for (int q = threadIdx.x; q < NH; q += 64 * kInferWaves) {
-        b1s[q] = w[OB1 + q];
-        b2s[q] = w[OB2 + q];
-        w3s[q] = bf2f(wq[NH * NI + NH * NH + q]);
-    }
-    const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
-    // W2 fragments: A[m = 16 mb + r][k = 16 s + 4 g + t]
-    bf16x4 f2[4][4];
+    const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4, wv = threadIdx.x >> 6;
+    // Wave wv takes lane group wv's inputs of W1 and block wv's rows of W2, 16
+    // bytes (two steps, or two groups of a step) per lane: four lanes read 64
+    // adjacent bytes, and 16 write adjacent slots.
+    static_assert(kInferWaves == 4, "one wave per lane group of W1 and per row block of W2");
+    uint4 p1[4], p2[2];
 #pragma unroll
     for (int mb = 0; mb < 4; ++mb)
+        p1[mb] = *reinterpret_cast<const uint4 *>(wq + (16 * mb + r) * NI + 32 * wv + 8 * g);
 #pragma unroll
-        for (int st = 0; st < 4; ++st)
-            f2[mb][st] = *reinterpret_cast<const bf16x4 *>(wq + NH * NI + (16 * mb + r) * NH +
-                                                          16 * st + 4 * g);
-    const float b3 = w[OB3];
-    __syncthreads();
+    for (int h = 0; h < 2; ++h)
+        p2[h] = *reinterpret_cast<const uint4 *>(wq + NH * NI + (16 * wv + r) * NH + 32 * h +
+                                                 8 * g);
     const int64_t ntiles = (n + 15) / 16;
     const int64_t nwaves = (int64_t)gridDim.x * kInferWaves;
-    int64_t tile = (int64_t)blockIdx.x * kInferWaves + (threadIdx.x >> 6);
+    int64_t tile = (int64_t)blockIdx.x * kInferWaves + wv;
     uint4 xv[4]; // this lane's 32 inputs of row 16 tile + r
     auto fetch = [&](int64_t tl) {
         const int64_t row = 16 * tl + r;
@@ -267,9 +264,31 @@ __global__ void __launch_bounds__(64 * kInferWaves)
                 xv[q] = src[q];
         }
     };
+    // the first tile's rows travel while the weights are staged
     if (tile < ntiles)
         fetch(tile);
+    const float b3 = w[OB3];
+#pragma unroll
+    for (int mb = 0; mb < 4; ++mb) {
+        bf16x4 *d = f1 + (mb * 8 + 2 * g) * 64 + wv * 16 + r;
+        d[0] = __builtin_bit_cast(bf16x4, ((uint64_t)p1[mb].y << 32) | p1[mb].x);
+        d[64] = __builtin_bit_cast(bf16x4, ((uint64_t)p1[mb].w << 32) | p1[mb].z);
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        bf16x4 *d = f2s + (wv * 4 + 2 * h + (g >> 1)) * 64 + 2 * (g & 1) * 16 + r;
+        d[0] = __builtin_bit_cast(bf16x4, ((uint64_t)p2[h].y << 32) | p2[h].x);
+        d[16] = __builtin_bit_cast(bf16x4, ((uint64_t)p2[h].w << 32) | p2[h].z);
+    }
+    for (int q = threadIdx.x; q < NH; q += 64 * kInferWaves) {
+        b1s[q] = w[OB1 + q];
+        b2s[q] = w[OB2 + q];
+        w3s[q] = bf2f(wq[NH * NI + NH * NH + q]);
+    }
+    __syncthreads();
     for (; tile < ntiles; tile += nwaves) {
+        int ln = lane; // opaque: known, the fragment reads are hoisted into registers
+        asm volatile("" : "+v"(ln));
         uint4 cur[4];
 #pragma unroll
         for (int q = 0; q < 4; ++q)
@@ -289,7 +308,7 @@ __global__ void __launch_bounds__(64 * kInferWaves)
             bx = __builtin_bit_cast(bf16x4, ((uint64_t)hi << 32) | lo);
 #pragma unroll
             for (int mb = 0; mb < 4; ++mb)
-                acc[mb] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(f1[(mb * 8 + st) * 64 + lane],
+                acc[mb] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(f1[(mb * 8 + st) * 64 + ln],
                                                                     bx, acc[mb], 0, 0, 0);
         }
         // bias + GELU, rounded to BF16: layer 2's B fragments
@@ -307,7 +326,8 @@ __global__ void __launch_bounds__(64 * kInferWaves)
             f32x4 a = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int st = 0; st < 4; ++st)
-                a = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(f2[mb][st], a1[st], a, 0, 0, 0);
+                a = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(f2s[(mb * 4 + st) * 64 + ln], a1[st],
+                                                           a, 0, 0, 0);
             acc[mb] = a;
         }
         // output layer on the BF16-rounded activations, then the 4 lane groups

@@ -52,6 +52,17 @@ def test_forward_matches_oracle(torch, orc, n):
     assert np.median(d) <= 1e-5 * scale, np.median(d)
 
 
+@pytest.mark.parametrize("n", [65, 4097, 16 * 4 * 1024 + 5, 196400])
+def test_forward_rows_are_independent(torch, n):
+    """One call over n rows equals calls over 1000 of them, bit for bit: the
+    last partial tile, and waves that take one, two and more tiles."""
+    print(f"[mlp forward rows] n={n}", flush=True)
+    m, _, X, _, _ = _setup(torch, 3, n)
+    got = m.forward(X)
+    ref = torch.cat([m.forward(X[i:i + 1000]) for i in range(0, n, 1000)])
+    assert torch.equal(got, ref)
+
+
 @pytest.mark.parametrize("n", [1, 33, 300])
 def test_gradient_matches_oracle(torch, orc, n):
     print(f"[mlp grad] n={n}", flush=True)
