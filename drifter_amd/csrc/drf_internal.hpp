@@ -191,7 +191,7 @@ template <class T> struct VolGeom {
 };
 
 // Resident workgroups per CU of each plain-RHS volume kernel, by [FP64 / FP32]
-// [128 / 256 / 512 lines][order][with the fused face phase]; set by the
+// [128 / 256 / 512 lines][order][with the faces]; set by the
 // kernel's first launch (0 before), read by the autotuner (api.cpp).
 extern int g_rhs_per_cu[2][3][kMaxN][2];
 

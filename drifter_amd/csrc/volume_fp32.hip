@@ -1,7 +1,8 @@
 // Volume right-hand side kernels, FP32 storage and arithmetic (mixed-precision
 // path; the free-surface column integrals stay FP64),
 // 128 grid lines per workgroup.  The kernel itself is in volume_impl.hpp; this
-// unit instantiates it for orders 1-8 and every fused epilogue.
+// unit instantiates the right-hand side and the whole Runge-Kutta steps for orders
+// 1-8.
 #include "volume_impl.hpp"
 
 namespace drf {

@@ -1,7 +1,7 @@
 // Volume right-hand side kernels, FP32 storage and arithmetic (mixed-precision
 // path; the free-surface column integrals stay FP64),
 // 256 grid lines per workgroup.  The kernel itself is in volume_impl.hpp; this
-// unit instantiates it for orders 1-4 and every fused epilogue.
+// unit instantiates the right-hand side for orders 1-4.
 #include "volume_impl.hpp"
 
 namespace drf {

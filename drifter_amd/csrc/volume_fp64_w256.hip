@@ -1,6 +1,6 @@
 // Volume right-hand side kernels, FP64 storage and arithmetic (parity path),
 // 256 grid lines per workgroup.  The kernel itself is in volume_impl.hpp; this
-// unit instantiates it for orders 1-4 and every fused epilogue.
+// unit instantiates the right-hand side for orders 1-4.
 #include "volume_impl.hpp"
 
 namespace drf {

@@ -208,8 +208,8 @@ drf_status drf_graph_rk(drf_ctx *ctx, int scheme, double dt, void *U, int layout
  * round trip: the maximum wave speed of U (compute_max_wave_speed, :153-168),
  * dt = AdaptiveTimeController::compute_dt(c, dx_min) (time_stepper.cpp:261-268)
  * written to dt_dev, time_dev += dt (time_ += dt_, :130; time_dev may be
- * NULL), then one fused step of `scheme` with that dt, which the stage
- * kernels read from dt_dev.  dt_dev, time_dev: device doubles.  FP64
+ * NULL), then one fused step of `scheme` with that dt, which the step
+ * kernel reads from dt_dev.  dt_dev, time_dev: device doubles.  FP64
  * contexts; fused schemes (not DP45).  Results equal drf_max_wave_speed_dev +
  * drf_compute_dt + drf_rk_step_dev(fused) bit for bit.  dx_min is the
  * driver's 2 / (N + 1) (:40-42). */
