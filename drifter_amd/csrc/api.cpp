@@ -67,19 +67,6 @@ drf_status ensure_work(drf_ctx *c, size_t bytes)
     return DRF_OK;
 }
 
-drf_status ensure_red(drf_ctx *c, int64_t len)
-{
-    if (c->red_len >= len)
-        return DRF_OK;
-    if (c->d_red)
-        DRF_HIP_CHECK(hipFree(c->d_red));
-    c->d_red = nullptr;
-    c->red_len = 0;
-    DRF_HIP_CHECK(hipMalloc(&c->d_red, sizeof(double) * len));
-    c->red_len = len;
-    return DRF_OK;
-}
-
 drf_status check_ready(const drf_ctx *c)
 {
     DRF_REQUIRE(c, DRF_ERR_ARG, "null context");
@@ -398,9 +385,6 @@ drf_status wave_speed(drf_ctx *c, const void *U, int layout, double *out, hipStr
     DRF_REQUIRE(c->precision == DRF_PREC_FP64, DRF_ERR_UNSUPPORTED,
                 "wave speed on the FP64 state only");
     const int64_t npart = wave_speed_parts(c->order, c->E);
-    drf_status st = ensure_red(c, npart + 1);
-    if (st)
-        return st;
     hipError_t e = launch_wave_speed(c->order, c->E, cview<double>(U, layout, c),
                                      coef_view<double>(c->d_h, c), c->d_red + 1, npart, s);
     if (e == hipSuccess)
@@ -422,9 +406,6 @@ drf_status adaptive_step(drf_ctx *c, int scheme, double cfl, double dx_min, doub
                          hipStream_t s)
 {
     const int64_t npart = wave_speed_parts(c->order, c->E);
-    drf_status st = ensure_red(c, npart + 1);
-    if (st)
-        return st;
     hipError_t e = launch_wave_speed(c->order, c->E, cview<double>(U, layout, c),
                                      coef_view<double>(c->d_h, c), c->d_red + 1, npart, s);
     if (e == hipSuccess)
@@ -607,6 +588,12 @@ drf_status drf_create(int order, int precision, int device, drf_ctx **out)
     if (e != hipSuccess) {
         delete c;
         return fail(DRF_ERR_HIP, std::string("hipStreamCreate: ") + hipGetErrorString(e));
+    }
+    e = hipMalloc(&c->d_red, sizeof(double) * (kMaxWaveParts + 1));
+    if (e != hipSuccess) {
+        (void)hipStreamDestroy(c->stream);
+        delete c;
+        return fail(DRF_ERR_HIP, std::string("reduction buffer: ") + hipGetErrorString(e));
     }
     *out = c;
     return DRF_OK;
@@ -955,10 +942,7 @@ drf_status drf_max_wave_speed_derived_dev(drf_ctx *c, const void *H, const void 
         return st;
     DRF_REQUIRE(H && u && v && c_max, DRF_ERR_ARG, "null argument");
     hipStream_t s = pick_stream(c, stream);
-    const int64_t npart = std::min<int64_t>(2048, (c->E + 3) / 4);
-    st = ensure_red(c, npart + 1);
-    if (st)
-        return st;
+    const int64_t npart = std::min<int64_t>(kMaxWaveParts, (c->E + 3) / 4);
     hipError_t e = launch_wave_speed_derived(c->order, c->E, (const double *)H, (const double *)u,
                                              (const double *)v, es, c->d_red + 1, npart, s);
     if (e == hipSuccess)
@@ -1041,10 +1025,6 @@ drf_status drf_graph_rk_adaptive(drf_ctx *c, int scheme, double cfl, double dx_m
     if (st)
         return st;
     DRF_REQUIRE(n_steps >= 1 && n_steps <= 100000, DRF_ERR_ARG, "n_steps must be 1..100000");
-    // the reduction buffer is the context's: size it before capturing
-    st = ensure_red(c, wave_speed_parts(c->order, c->E) + 1);
-    if (st)
-        return st;
     return capture_graph(c, 0, n_steps, out, [&](hipStream_t cs) {
         return adaptive_step(c, scheme, cfl, dx_min, dt_min, dt_max, U, layout,
                              (double *)dt_dev, (double *)time_dev, cs);

@@ -240,13 +240,16 @@ inline hipError_t launch_volume_fp32(int order, const VolGeom<float> &geo, const
 }
 
 // Vector kernels (stepper.hip)
-// Workgroups (partial maxima) of the wave-speed reduction: at most 2048, each
-// with the same number of batches of 256 / (N + 1)^2 elements but the last
-// (2048 workgroups on 3,277 batches ran 2 rounds for 1.6 rounds' work).
+// Workgroups (partial maxima) of a wave-speed reduction at most: the length of
+// every buffer that takes them.
+constexpr int64_t kMaxWaveParts = 2048;
+// Workgroups of the reduction over a state, each with the same number of
+// batches of 256 / (N + 1)^2 elements but the last (2048 workgroups on 3,277
+// batches ran 2 rounds for 1.6 rounds' work).
 inline int64_t wave_speed_parts(int order, int64_t E)
 {
     const int64_t epb = 256 / ((order + 1) * (order + 1)), nb = (E + epb - 1) / epb;
-    const int64_t rounds = (nb + 2047) / 2048;
+    const int64_t rounds = (nb + kMaxWaveParts - 1) / kMaxWaveParts;
     return (nb + rounds - 1) / rounds;
 }
 hipError_t launch_wave_speed(int order, int64_t E, View<const double> U, View<const double> h,
@@ -299,8 +302,9 @@ struct drf_ctx {
     // host-packed staging and RK work space (grown on demand)
     void *d_work = nullptr;
     size_t work_bytes = 0;
-    double *d_red = nullptr; // reduction scratch
-    int64_t red_len = 0;
+    // wave-speed reduction: the maximum, then kMaxWaveParts partials.  Allocated
+    // with the context and never moved, as captured graphs hold its address.
+    double *d_red = nullptr;
     // volume-kernel launch shape (drf_set_launch / drf_autotune)
     int wg_per_cu = 0;
     int xcd_remap = 1;

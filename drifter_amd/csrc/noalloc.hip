@@ -1,8 +1,7 @@
 // The CFL wave-speed maximum with no device allocation: the partial maxima
-// of the reduction live in a file-scope device array instead of the
-// context's lazily allocated reduction buffer, and the maximum is written to
-// a device double the caller owns.  For callers that cannot allocate (code
-// under HIP graph capture, serving loops that forbid hipMalloc).
+// of the reduction live in a file-scope device array instead of the context's
+// reduction buffer, and the maximum is written to a device double the caller
+// owns.  For callers that cannot synchronise (code under HIP graph capture).
 //
 // `scratch` is one array per GPU, held until the process ends; every call on
 // a GPU shares it, so calls that overlap on one GPU race.  Each call writes
@@ -13,14 +12,7 @@
 
 #include "drf_internal.hpp"
 
-namespace drf {
-
-// at most this many partial maxima (the wave-speed launch never uses more)
-constexpr int64_t kScratchPartials = 2048;
-
-} // namespace drf
-
-static __device__ __align__(256) double scratch[drf::kScratchPartials];
+static __device__ __align__(256) double scratch[drf::kMaxWaveParts];
 
 namespace drf {
 namespace {
@@ -73,10 +65,10 @@ extern "C" drf_status drf_max_wave_speed_noalloc_dev(drf_ctx *c, const void *U, 
                     "drf_max_wave_speed_noalloc_dev: wave speed on the FP64 state only");
     // the same partial count as drf_max_wave_speed_dev, so the two agree bit for bit
     const int64_t npart = wave_speed_parts(c->order, c->E);
-    if (npart > kScratchPartials)
+    if (npart > kMaxWaveParts)
         return fail(DRF_ERR_ARG, "drf_max_wave_speed_noalloc_dev: " + std::to_string(npart) +
                                      " partial maxima exceed the scratch array's " +
-                                     std::to_string(kScratchPartials));
+                                     std::to_string(kMaxWaveParts));
     double *part = scratch_ptr(c->device);
     if (!part)
         return fail(DRF_ERR_STATE,

@@ -104,6 +104,42 @@ def test_graph_of_adaptive_steps_replays_exactly():
         assert tg.item() == te.item() and dtg.item() == dte.item(), rep
 
 
+@pytest.mark.parametrize("order,E", [(3, 256), (1, 125), (4, 333)])
+def test_graph_survives_wave_speeds_of_derived_arrays(orc, order, E):
+    """A captured graph keeps the address of the context's reduction buffer.
+    The wave speed of derived arrays reduces more partials than the state's
+    (64 against 16 on the first mesh); called between the replays, with device
+    memory allocated and filled around it, it must not move that buffer."""
+    import torch
+
+    layout = _lib.LAYOUT_SOA
+    print(f"[adaptive] graph, derived wave speed between replays, N={order} E={E}", flush=True)
+    case = synth.make_case(8, 8, 6, order, 10000.0, "seamount")
+    h, P = case.h[:E * case.nd], case.U[:E * 5 * case.nd]
+    s = PrimitiveEquationsSolver(order)
+    s.initialize(E, h, coriolis=CoriolisParameter(1e-4, 0.0, 0.0))
+    U = torch.from_numpy(synth.to_soa(P, E, case.nd)).cuda()
+    H, u, v, _, _ = orc.derived(order, P, h)
+    want = orc.max_wave_speed(order, H, u, v)
+    D = [torch.from_numpy(a).cuda() for a in (H, u, v)]
+    Ue = U.clone()
+    dte, te, dtg, tg = (torch.zeros(1, dtype=torch.float64, device="cuda") for _ in range(4))
+    g = s.capture_adaptive_steps(_lib.RK_RK4, U, dtg, tg, n_steps=2, cfl=CFL, dt_min=DT_MIN,
+                                 dt_max=DT_MAX, layout=layout)
+    keep = []
+    for rep in range(3):
+        assert s.max_wave_speed_derived_dev(*D, case.nd) == want
+        keep.append(torch.full((100000,), 1e30, dtype=torch.float64, device="cuda"))
+        for _ in range(2):
+            s.rk_step_adaptive_dev(_lib.RK_RK4, Ue, dte, te, cfl=CFL, dt_min=DT_MIN,
+                                   dt_max=DT_MAX, layout=layout)
+        torch.cuda.synchronize()
+        g.launch()
+        torch.cuda.synchronize()
+        assert torch.equal(U, Ue), rep
+        assert tg.item() == te.item() and dtg.item() == dte.item(), rep
+
+
 def test_one_adaptive_step_matches_the_oracle(orc):
     import torch
 
