@@ -310,14 +310,21 @@ __device__ __forceinline__ void load_f(Lines<n, TC> &L, const VolGeom<TS> &geo, 
     }
 }
 
-// Fields [F0, F0 + NFD) of the xi-line at offset so into u[0..]
-template <int n, int F0, int NFD, bool ADJ, class TS, class TC, int NU>
+// Fields [F0, F0 + NFD) of the xi-line at offset so into u[0..], node by node
+// or (BY_FIELD) field by field
+template <int n, int F0, int NFD, bool ADJ, bool BY_FIELD = false, class TS, class TC, int NU>
 __device__ __forceinline__ void load_fields(const View<const TS> &U, uint32_t so, TC (&u)[NU][n])
 {
     if constexpr (ADJ) {
 #pragma unroll
         for (int f = 0; f < NFD; ++f)
             ld_run<n, TS, TC>(U.p + (F0 + f) * U.fs, so, u[f]);
+    } else if constexpr (BY_FIELD) {
+#pragma unroll
+        for (int f = 0; f < NFD; ++f)
+#pragma unroll
+            for (int i = 0; i < n; ++i)
+                u[f][i] = ldo<TS, TC>(U.p + (F0 + f) * U.fs + i * U.is, so);
     } else {
 #pragma unroll
         for (int i = 0; i < n; ++i)
@@ -326,6 +333,13 @@ __device__ __forceinline__ void load_fields(const View<const TS> &U, uint32_t so
                 u[f][i] = ldo<TS, TC>(U.p + (F0 + f) * U.fs + i * U.is, so);
     }
 }
+
+// Plain right-hand sides whose lines fill the registers (FP64 from N = 5, FP32
+// at N = 8) load a node's bathymetry with its fields and take the LDS places of
+// their lines from outside the phases: 4 M nodes, FP64 N = 6 133.4 -> 130.6, N =
+// 7 118.0 -> 115.3, mixed N = 8 93.4 -> 90.2 us.  The others were the same or
+// slower (mixed N = 6 56.8 -> 57.6, FP64 N = 4 83.7 -> 84.0 us).
+template <int n, class TC> constexpr bool wide_line() { return sizeof(TC) == 8 ? n >= 6 : n == 9; }
 
 // All of P1's global loads are issued here, so that P1 itself waits only for
 // them: a load issued inside P1 would make the wave wait for every store of
@@ -336,8 +350,21 @@ __device__ __forceinline__ void load_lines(Lines<n, TC> &L, const View<const TS>
                                            const VolGeom<TS> &geo, int64_t b, int64_t e, int line)
 {
     const uint32_t uo = state_off<EPB>(U, b, e, line);
-    load_fields<n, 0, NF, ADJ>(U, uo, L.q);
-    load_h<n, TS, TC>(L, geo, e, line);
+    if constexpr (WITH_F && !ADJ && wide_line<n, TC>()) {
+        // a node's bathymetry with its fields, as P1 takes both node by node:
+        // with h last P1 waited for the whole line
+        const uint32_t ho = flat_off(geo.h, e, line);
+#pragma unroll
+        for (int i = 0; i < n; ++i) {
+#pragma unroll
+            for (int f = 0; f < NF; ++f)
+                L.q[f][i] = ldo<TS, TC>(U.p + f * U.fs + i * U.is, uo);
+            L.hb[i] = ldo<TS, TC>(geo.h.p + i * geo.h.is, ho);
+        }
+    } else {
+        load_fields<n, 0, NF, ADJ>(U, uo, L.q);
+        load_h<n, TS, TC>(L, geo, e, line);
+    }
     if (WITH_F)
         load_f<n, TS, TC>(L, geo, e, line);
 }
@@ -658,6 +685,7 @@ __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_wav
     // The right-hand side prefetches the next batch's lines.  A Runge-Kutta
     // step keeps its stage state, initial state and accumulator in those
     // registers instead, and runs every stage of one batch before the next.
+    constexpr int n = C::n;
     constexpr bool STEP = EPI != EPI_RHS;
     constexpr bool PREFETCH = !STEP;
     // With faces FP64 at N = 4 has no registers to prefetch the tracers, which
@@ -671,7 +699,20 @@ __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_wav
     // FP64 from N = 6 has no registers to load a step's initial state a phase
     // early (SSP-RK3 at N = 8: 555 us early, 544 us at the use)
     constexpr bool LATE = sizeof(TC) == 8 && N >= 6;
-    constexpr int n = C::n, n2 = C::n2, n3 = C::n3, EPB = C::EPB;
+    // ... and then field by field where that was the faster order: 4 M nodes,
+    // node by node and field by field, Euler N = 6 148.7 and 147.2, N = 8 219.8
+    // and 213.5 us, RK4 N = 6 426 and 400, N = 8 675 and 666 us, SSP-RK3 N = 8
+    // 542 and 523 us, but N = 7 301 and 306 us.
+    constexpr bool BY_FIELD = LATE && N != 7;
+    constexpr bool PLACES_OUTSIDE = !STEP && FACES == FACES_NONE && wide_line<n, TC>();
+    // The plain right-hand side's phases stand in a loop of one trip where the
+    // compiler then keeps fewer bases and operators live across them (4 M nodes,
+    // straight and in the loop: FP64 N = 6 133 and 113 us; FP32 N = 2 48.2 and
+    // 44.2, N = 3 42.4 and 41.0 us); it was slower at every other order (FP64
+    // N = 5 85 and 93, FP32 N = 4 46.5 and 50.3, N = 7 56 and 79 us).
+    constexpr bool ONE_TRIP = !STEP && FACES == FACES_NONE &&
+                              (sizeof(TC) == 8 ? N == 6 : N == 2 || N == 3);
+    constexpr int n2 = C::n2, n3 = C::n3, EPB = C::EPB;
     using P = Place<n, (int)sizeof(TC)>;
     __shared__ TC sm[EPB * P::ES];
     // column integrals, double-buffered by batch parity: the last phase of
@@ -774,18 +815,23 @@ __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_wav
                 for (int i = 0; i < n; ++i)
                     acc[f][i] = (TC)0;
         }
-        // One evaluation of the right-hand side of cur (a lambda and no loop
-        // around the phases for the plain right-hand side: a loop of one trip
-        // cost it 35 VGPRs at N = 3).
+        // nodes of the xi-, eta- and zeta-line in slot 0
+        TC *rx = nullptr, *ry = nullptr, *rz = nullptr;
+        if constexpr (PLACES_OUTSIDE) {
+            rx = sm + le * P::ES + (L0 % n) * P::SJ + (L0 / n) * P::SK;
+            ry = sm + (lines & 0xffffu);
+            rz = sm + (lines >> 16);
+        }
+        // One evaluation of the right-hand side of cur.
         auto evaluate = [&](int st) __attribute__((always_inline)) {
         // In a step the line is opaque to the compiler, so that it hoists no
         // load or address out of the stages into registers they do not have.
         int L = L0;
         if constexpr (STEP)
             asm volatile("" : "+v"(L));
-        // nodes of the xi-, eta- and zeta-line in slot 0
-        TC *sx = sm + le * P::ES + (L % n) * P::SJ + (L / n) * P::SK;
-        TC *sy = sm + (lines & 0xffffu), *sz = sm + (lines >> 16);
+        TC *sx = PLACES_OUTSIDE ? rx : sm + le * P::ES + (L % n) * P::SJ + (L / n) * P::SK;
+        TC *sy = PLACES_OUTSIDE ? ry : sm + (lines & 0xffffu),
+           *sz = PLACES_OUTSIDE ? rz : sm + (lines >> 16);
         const StageCoefs<TC> sc = stage_coefs<TS, TC>(epi, st);
 
         // Register state carried by the xi-owner: the momentum partials
@@ -941,7 +987,7 @@ __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_wav
         // ---------------- P3a: zeta-line (i, j) = L, momentum ----------------
         TC um[2][n]; // initial Hu, Hv for P4a
         if constexpr (step_reads_u0(EPI) && !LATE)
-            load_fields<n, 0, 2, ADJ>(U, state_off<EPB>(U, b, e, L), um);
+            load_fields<n, 0, 2, ADJ, BY_FIELD>(U, state_off<EPB>(U, b, e, L), um);
         {
             TC u[n], v[n], hi[n];
 #pragma unroll
@@ -973,7 +1019,7 @@ __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_wav
                 kv[1][i] = pHv[i] + sx[S_B * P::SS + i];
             }
             if constexpr (step_reads_u0(EPI) && LATE)
-                load_fields<n, 0, 2, ADJ>(U, state_off<EPB>(U, b, e, L), um);
+                load_fields<n, 0, 2, ADJ, BY_FIELD>(U, state_off<EPB>(U, b, e, L), um);
             if constexpr (STEP)
                 stage_update<n, 0, 2, EPI>(sc, kv, um, cur.q, acc);
             else
@@ -1021,7 +1067,7 @@ __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_wav
         // threads touch the same node of the same slot.
         TC ut[3][n]; // initial eta, HT, HS for P4b
         if constexpr (step_reads_u0(EPI) && !LATE)
-            load_fields<n, 2, 3, ADJ>(U, state_off<EPB>(U, b, e, L), ut);
+            load_fields<n, 2, 3, ADJ, BY_FIELD>(U, state_off<EPB>(U, b, e, L), ut);
         {
             TC ftv[n], fsv[n];
 #pragma unroll
@@ -1080,7 +1126,7 @@ __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_wav
                 kv[2][i] = (pHS[i] + sx[S_B * P::SS + i]) + sx[S_D * P::SS + i];
             }
             if constexpr (step_reads_u0(EPI) && LATE)
-                load_fields<n, 2, 3, ADJ>(U, state_off<EPB>(U, b, e, L), ut);
+                load_fields<n, 2, 3, ADJ, BY_FIELD>(U, state_off<EPB>(U, b, e, L), ut);
             if constexpr (STEP)
                 stage_update<n, 2, 3, EPI>(sc, kv, ut, cur.q, acc);
             else
@@ -1098,6 +1144,10 @@ __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_wav
         if constexpr (STEP) {
 #pragma unroll 1
             for (int st = 0; st < epi.nst; ++st)
+                evaluate(st);
+        } else if constexpr (ONE_TRIP) {
+#pragma unroll 1
+            for (int st = 0; st < 1; ++st)
                 evaluate(st);
         } else {
             evaluate(0);

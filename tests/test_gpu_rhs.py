@@ -111,7 +111,7 @@ def test_error_before_initialize():
     s.close()
 
 
-@pytest.mark.parametrize("order", [3, 4, 1])
+@pytest.mark.parametrize("order", [3, 4, 1, 2])
 @pytest.mark.parametrize("prec", [_lib.PREC_FP64, _lib.PREC_MIXED])
 def test_launch_shape_does_not_change_results(prec, order):
     """every element is computed the same way whatever the grid: all launch
