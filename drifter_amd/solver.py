@@ -62,12 +62,16 @@ def _sptr(s):
     """HIP stream handle: a torch stream, an int handle, or torch's current
     stream when None (so device calls are ordered after torch's copies).  The
     current stream's handle is asked for directly: building torch's Stream
-    object took 2.7 of a small call's 9 us."""
+    object took 2.7 of a small call's 9 us.  torch's functions for that are not
+    public: a torch without them takes the Stream object."""
     if s is None:
         import torch
 
         if torch.cuda.is_initialized():
-            return C.c_void_p(torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice()))
+            try:
+                return C.c_void_p(torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice()))
+            except AttributeError:
+                pass
         s = torch.cuda.current_stream()
     if hasattr(s, "cuda_stream"):
         return C.c_void_p(s.cuda_stream)
