@@ -3,11 +3,15 @@ against the same scheme composed of right-hand sides and vector updates, at
 every order, precision and layout, on element counts around one workgroup's
 batch (128 grid lines: 128 // (N + 1)^2 elements) and past it.
 
-Tolerance: both sides evaluate the same expressions; they differ in FMA
-contraction only.  Each stage's combination rounds a few times at the size of
-the state (8 eps of the field's maximum covers five stages), and a tendency's
-rounding enters multiplied by dt (a contraction of n terms of operands up to
-the largest |D| ~ n^2: 1e-12 of the largest tendency in FP64, 1e-4 in FP32).
+Tolerance, field by field: both sides evaluate the same expressions and differ
+in FMA contraction and in the rounding of the stage states.  A stage's
+combination rounds a few times at the size of the field, and a rounding of the
+stage state by eps |U| or of a contraction's terms moves the field's tendency by
+eps times the size of its terms (_term_size: the largest row sum of |D| times
+the fluxes, the pressure gradient and the diffusion), which enters times dt: 8
+eps (max |U_f| + stages dt terms_f).  dt is half the CFL step, so that every
+field's update and, against the Euler step, some field's stages exceed that
+tolerance many times; both are asserted.
 """
 import numpy as np
 import pytest
@@ -45,6 +49,38 @@ def _composed(k, U, scheme, dt):
     return Y
 
 
+STAGES = {"euler": 1, "rk2": 2, "ssprk3": 3, "rk4": 4, "lsrk45": 5}
+
+
+def _fields(V, layout, E, n, block):
+    """The flat state as (E, 5, nd) float64 on the host."""
+    A = V.double().cpu().numpy()
+    if layout == _lib.LAYOUT_SOA:
+        A = synth.from_soa(A, E, n ** 3)
+    elif layout == _lib.LAYOUT_LINES:
+        A = synth.from_lines(A, E, n)
+    elif layout == _lib.LAYOUT_BLOCKS:
+        A = synth.from_blocks(A, E, n, block)
+    return A.reshape(E, 5, n ** 3)
+
+
+def _term_size(P, h, order):
+    """Sizes of the terms of each field's tendency, and half the CFL step."""
+    n = order + 1
+    D = np.zeros(n * n)
+    _lib.load().drf_basis(order, None, None, _lib.dptr(D))
+    row = np.abs(D).reshape(n, n).sum(axis=1).max()
+    H = P[:, 2] + h
+    Hm = np.abs(H).max()
+    q = np.abs(P).max(axis=(0, 2))
+    u, v = np.abs(P[:, 0] / H).max(), np.abs(P[:, 1] / H).max()
+    grad = 9.81 * Hm * row * q[2]  # g H times a derivative of eta
+    terms = np.array([row * q[0] * (u + v) + grad + 2 * Hm * row ** 2 * u,
+                      row * q[1] * (u + v) + grad + 2 * Hm * row ** 2 * v,
+                      row * (q[0] + q[1]), row * q[3] * (u + v), row * q[4] * (u + v)])
+    return terms, 0.5 * (2.0 / n) / (np.sqrt(9.81 * Hm) + max(u, v))
+
+
 @pytest.mark.parametrize("order", range(1, 9))
 @pytest.mark.parametrize("prec", [_lib.PREC_FP64, _lib.PREC_MIXED])
 @pytest.mark.parametrize("scheme", sorted(SCHEMES))
@@ -53,10 +89,10 @@ def test_step_is_the_composed_scheme(order, prec, scheme):
 
     n = order + 1
     batch = max(1, 128 // (n * n))
+    block = _lib.load().drf_layout_block_elements(order)
     full = synth.make_case(5, 5, 8, order, 10000.0, "seamount")
     nd, dtype = n ** 3, torch.float64 if prec == _lib.PREC_FP64 else torch.float32
     eps = float(np.finfo(np.float64 if prec == _lib.PREC_FP64 else np.float32).eps)
-    dt = 1e-3
     for q, E in enumerate(sorted({1, max(1, batch - 1), batch, batch + 1, 3 * batch + 2})):
         E = min(E, full.E)
         layout = LAYOUTS[(q + order) % 4]
@@ -66,12 +102,13 @@ def test_step_is_the_composed_scheme(order, prec, scheme):
         s.initialize(E, full.h[:E * nd], coriolis=CoriolisParameter(1e-4, beta, 0.0),
                      y_positions=full.y[:E * nd])
         P = full.U[:E * 5 * nd]
+        terms, dt = _term_size(P.reshape(E, 5, nd), full.h[:E * nd].reshape(E, nd), order)
         if layout == _lib.LAYOUT_SOA:
             P = synth.to_soa(P, E, nd)
         elif layout == _lib.LAYOUT_LINES:
             P = synth.to_lines(P, E, n)
         elif layout == _lib.LAYOUT_BLOCKS:
-            P = synth.to_blocks(P, E, n, _lib.load().drf_layout_block_elements(order))
+            P = synth.to_blocks(P, E, n, block)
         U = torch.from_numpy(np.ascontiguousarray(P)).cuda().to(dtype)
 
         def k(V):
@@ -80,12 +117,20 @@ def test_step_is_the_composed_scheme(order, prec, scheme):
             return R
 
         want = _composed(k, U, scheme, dt)
-        rate = float(k(U).abs().max())
+        euler = _composed(k, U, "euler", dt)
         got = U.clone()
         s.rk_step_dev(SCHEMES[scheme], 0.0, dt, got, layout)
         torch.cuda.synchronize()
-        tol = 8 * eps * float(U.abs().max()) + dt * (1e-12 if eps < 1e-12 else 1e-4) * rate
-        assert float((got - want).abs().max()) <= tol
+        W, A, B, G = (_fields(V, layout, E, n, block) for V in (want, U, euler, got))
+        size = np.abs(A).max(axis=(0, 2))
+        tol = 8 * eps * (size + STAGES[scheme] * dt * terms)
+        err = np.abs(G - W).max(axis=(0, 2)) / tol
+        print("  error / tolerance", np.round(err, 3), flush=True)
+        assert (err <= 1.0).all(), err
+        # what the tolerance tells apart
+        assert (np.abs(W - A).max(axis=(0, 2)) >= 20 * tol).all()
+        if scheme != "euler":
+            assert (np.abs(W - B).max(axis=(0, 2)) / tol).max() >= 10.0
         s.close()
 
 
