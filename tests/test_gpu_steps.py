@@ -134,6 +134,46 @@ def test_step_is_the_composed_scheme(order, prec, scheme):
         s.close()
 
 
+@pytest.mark.parametrize("order,mesh,E", [(6, (32, 16, 16), 6145), (7, (16, 16, 16), 4095),
+                                          (8, (16, 16, 16), 3331)])
+@pytest.mark.parametrize("layout", [_lib.LAYOUT_PACKED, _lib.LAYOUT_LINES])
+def test_steps_of_resident_workgroups(order, mesh, E, layout):
+    """FP64 steps from order 6 run resident workgroups that loop over several
+    batches each, in place, on meshes of more batches than fit the card at once.
+    The right-hand side is element-local: the step equals, bit for bit, steps of
+    300 of the elements at a time, whose batches get a workgroup each.  A
+    workgroup holds two elements at orders 6 and 7 and one at order 8, and at
+    most four fit a CU, so the batches fill the card three times and the last
+    one is part-filled."""
+    import torch
+
+    n, nd = order + 1, (order + 1) ** 3
+    full = synth.make_case(*mesh, order, 10000.0, "seamount")
+    assert full.E >= E
+    h = full.h[:E * nd]
+    P = torch.from_numpy(full.U[:E * 5 * nd].reshape(E, 5, n * n, n)).cuda()
+
+    def flat(V):
+        return V.permute(1, 3, 0, 2).contiguous() if layout == _lib.LAYOUT_LINES else V.clone()
+
+    def step(V, hs, scheme):
+        s = PrimitiveEquationsSolver(order)
+        s.initialize(V.shape[0], hs, coriolis=CoriolisParameter(1e-4, 0.0, 0.0))
+        U = flat(V)
+        s.rk_step_dev(SCHEMES[scheme], 0.0, 2e-3, U.view(-1), layout)
+        torch.cuda.synchronize()
+        s.close()
+        return U.permute(2, 0, 3, 1) if layout == _lib.LAYOUT_LINES else U
+
+    for scheme in sorted(SCHEMES):
+        print(f"[resident steps] order={order} E={E} layout={layout} {scheme}", flush=True)
+        got = step(P, h, scheme)
+        for e in range(0, E, 300):
+            c = slice(e, min(E, e + 300))
+            assert torch.equal(got[c], step(P[c], h[c.start * nd:c.stop * nd], scheme)), e
+        assert not torch.equal(got, P)
+
+
 @pytest.mark.parametrize("order,E", [(1, 64 * 3 + 1), (2, 27), (3, 16 * 2049 + 3), (4, 10 * 2048),
                                      (6, 11), (8, 3 * 2048 + 1)])
 @pytest.mark.parametrize("layout", [_lib.LAYOUT_SOA, _lib.LAYOUT_LINES])
