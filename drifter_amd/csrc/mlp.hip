@@ -477,9 +477,10 @@ __global__ void __launch_bounds__(256)
     }
 }
 
-// Sum of the partial gradients (fixed order), then either write the
-// gradient or take one Adam step on the master weights and refresh their
-// BF16 copies.  A workgroup takes 64 parameters, its wavefronts a quarter of
+// Sum of the partial gradients (fixed order, in FP64: small batches have
+// twice the partials that tiles of 32 rows gave, and the FP32 sum's error grew
+// with them; the time is the same), then either write the gradient or take one
+// Adam step on the master weights and refresh their BF16 copies.  A workgroup takes 64 parameters, its wavefronts a quarter of
 // the partials each: with one thread for a parameter's whole sum the kernel
 // was that sum's chain of loads on 49 workgroups (64 partials: 4.9 us, now
 // 3.7 us).
@@ -489,33 +490,34 @@ __global__ void __launch_bounds__(256)
                       float *__restrict__ loss, AdamStep adam, float *__restrict__ w,
                       float *__restrict__ m, float *__restrict__ v, uint16_t *__restrict__ wq)
 {
-    __shared__ float quarter[4][64];
+    __shared__ double quarter[4][64];
     const int lane = threadIdx.x & 63, part = threadIdx.x >> 6;
     const int p = blockIdx.x * 64 + lane;
     const int per = (nparts + 3) / 4, first = part * per;
     const int last = first + per < nparts ? first + per : nparts;
-    float g = 0.f;
+    double q = 0.0;
     if (p < NP) {
 #pragma unroll 16
         for (int i = first; i < last; ++i)
-            g += partial[(size_t)i * NP + p];
+            q += (double)partial[(size_t)i * NP + p];
     }
-    quarter[part][lane] = g;
+    quarter[part][lane] = q;
     // the loss: lane sums of every 64th partial, then the lanes
     if (blockIdx.x == 0 && part == 1 && loss) {
-        float a = 0.f;
+        double a = 0.0;
         for (int i = lane; i < nparts; i += 64)
-            a += lpart[i];
+            a += (double)lpart[i];
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1)
             a += __shfl_xor(a, o);
         if (lane == 0)
-            *loss = a * inv_b;
+            *loss = (float)(a * (double)inv_b);
     }
     __syncthreads();
     if (part != 0 || p >= NP)
         return;
-    g = quarter[0][lane] + quarter[1][lane] + quarter[2][lane] + quarter[3][lane];
+    const float g = (float)(quarter[0][lane] + quarter[1][lane] + quarter[2][lane] +
+                            quarter[3][lane]);
     if (grad)
         grad[p] = g;
     if (adam.lr != 0.f) {

@@ -79,6 +79,29 @@ def test_gradient_matches_oracle(torch, orc, n):
         assert err <= 1e-2, (name, err)
 
 
+@pytest.mark.parametrize("n", [256, 2048, 4096])
+def test_gradient_is_the_sum_of_its_tiles(torch, n):
+    """A batch of 2^k rows up to 4096 takes tiles of 16 rows.  Its gradient and
+    loss are 16 / n times the sums over those of the tiles alone: scaling by a
+    power of two is exact in every product and rounding, so only that sum
+    rounds.  It is formed in 64 bits and rounded once: half a unit in the last
+    place of the result, and 1e-15 of the terms for the order of the sum."""
+    print(f"[mlp tiles] n={n}", flush=True)
+    m, _, X, _, y = _setup(torch, 7, n)
+    yt = torch.from_numpy(y).cuda()
+    loss, grad = m.loss_grad(X, yt)
+    g, l = [], []
+    for r in range(0, n, 16):
+        a, b = m.loss_grad(X[r:r + 16], yt[r:r + 16])
+        l.append(a.double())
+        g.append(b.double())
+    for got, parts in ((grad, torch.stack(g)), (loss, torch.stack(l))):
+        parts = parts * (16.0 / n)
+        want = parts.sum(dim=0)
+        tol = 2.0 ** -24 * (1 + 1e-6) * want.abs() + 1e-15 * parts.abs().sum(dim=0)
+        assert ((got.double() - want).abs() <= tol).all()
+
+
 def test_gradient_deterministic(torch):
     m, p, X, Xf, y = _setup(torch, 5, 5000)
     yt = torch.from_numpy(y).cuda()
