@@ -39,8 +39,9 @@ struct drf_face_plan {
     std::vector<int64_t> conf; // [nc][4]: left element, left face, right element, right face
     std::vector<int64_t> mort; // [nm][6]: coarse element, coarse face, fine elements by sub-face
     std::vector<int> mort_type;
-    // [E][6]: (neighbour << 4) | (neighbour's face << 1) | side of every
-    // conforming face (side 0: the element is the interface's left), else -1
+    // [E][6]: (neighbour << 1) | side of every conforming face (side 0: the
+    // element is the interface's left; the neighbour's face is f ^ 1), else all
+    // ones: 31 bits for the neighbour
     std::vector<uint32_t> eface;
     int64_t *d_conf = nullptr, *d_mort = nullptr;
     uint32_t *d_eface = nullptr;
@@ -274,6 +275,8 @@ drf_status drf_face_plan_create(const drf_ctx *ctx, int64_t n_elem, const double
                 "drf_face_plan_create: context not initialized");
     DRF_REQUIRE(n_elem == ctx->E, DRF_ERR_ARG,
                 "drf_face_plan_create: element count differs from the context's");
+    DRF_REQUIRE(n_elem < (int64_t(1) << 31), DRF_ERR_UNSUPPORTED,
+                "drf_face_plan_create: more than 2^31 - 1 elements");
     DRF_REQUIRE(ctx->n >= 2 && ctx->n <= 5, DRF_ERR_UNSUPPORTED,
                 "drf_face_plan_create: face kernels are built for orders 1-4");
     DRF_REQUIRE(bounds && levels && type && count && elems && faces, DRF_ERR_ARG,
