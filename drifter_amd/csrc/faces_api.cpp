@@ -240,6 +240,11 @@ template <class T> bool volume_faces(const drf_face_plan *p, int layout, VolFace
     fill_args<T>(p, a, nullptr, nullptr, layout);
     if (!element_offsets_fit<T>(p, a))
         return false;
+    // the fused flux takes the velocity along the face's axis only, where the
+    // components' has the other two times zero: not the same if they are not finite
+    for (int i = 0; i < 4; ++i)
+        if (!std::isfinite(a.p[i]))
+            return false;
     out->eface = p->d_eface;
     out->wq = (const T *)p->d_wq;
     for (int i = 0; i < 4; ++i)

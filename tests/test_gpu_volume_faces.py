@@ -66,3 +66,34 @@ def test_volume_faces_are_the_element_launch(order, prec, kind, params):
     plan.detach()
     plan.close()
     s.close()
+
+
+@pytest.mark.parametrize("kind", [faces.LF_ADV, faces.UPWIND])
+def test_parameters_that_are_not_finite(kind):
+    """v n of the scalar fluxes sums all three axes, so one infinite velocity
+    makes every face's flux NaN, in the volume kernel as in the element launch."""
+    import torch
+
+    print(f"[volume faces] infinite velocity kind={kind}", flush=True)
+    m = OctreeAdapter(0.0, 10000.0, 0.0, 10000.0, -1.0, 0.0)
+    m.build_uniform(4, 4, 2)
+    bounds, levels, _ = m.elements()
+    case = synth.make_case_on(bounds, 2, 10000.0, "seamount")
+    s = PrimitiveEquationsSolver(2)
+    s.initialize(case.E, case.h, coriolis=CoriolisParameter(1e-4, 0.0, 0.0))
+    plan = faces.FacePlan(s, bounds, levels, m.build_face_connections(two_to_one=True), kind=kind,
+                          params=(0.3, float("inf"), 0.1, 0.6))
+    plan.attach()
+    U = torch.from_numpy(np.ascontiguousarray(_state(case, "lines"))).cuda()
+    out = []
+    for mode in (faces.BY_ELEMENT, faces.IN_VOLUME):
+        plan.set_conforming_mode(mode)
+        out.append(torch.zeros_like(U))
+        s.compute_rhs_dev(U, out[-1], _lib.LAYOUT_LINES)
+    torch.cuda.synchronize()
+    assert torch.isnan(out[0]).any()
+    assert torch.equal(torch.isnan(out[0]), torch.isnan(out[1]))
+    assert torch.equal(torch.nan_to_num(out[0]), torch.nan_to_num(out[1]))
+    plan.detach()
+    plan.close()
+    s.close()
