@@ -615,12 +615,24 @@ template <int n, int NFD, class T> struct FaceNodes {
 };
 
 // Fields whose neighbour nodes are in flight at once: all where the registers
-// allow it, else one chunk while the next one loads (39,280 elements: FP64
-// N = 3 all 102, one by one 106 us, N = 4 one by one 206, in twos 220 us; FP32
-// N = 4 in twos 116, one by one 121, all 128 us).
-template <int N, class T> constexpr int face_chunk()
+// allow it, else one chunk while the next one loads.  Coastline octree, 39,280
+// elements, line layout, LF / UPWIND, in us, and the VGPRs spilled at N = 4:
+//              all at once      in twos          one by one
+//   FP64 N = 1  26.0 /  25.9    25.7 /  25.7     26.1 /  26.0
+//   FP64 N = 2  49.2 /  48.1    48.6 /  47.8     50.8 /  51.4
+//   FP64 N = 3  96.4 /  95.7    96.4 /  96.3    100.8 / 100.0
+//   FP64 N = 4   293 /   287 (53)  219 / 249 (28)  212 / 207 (5)
+//   FP32 N = 1  21.8 /  21.7    21.0 /  21.0     21.3 /  21.3
+//   FP32 N = 2  32.8 /  32.4    33.0 /  33.6     35.4 /  35.8
+//   FP32 N = 3  53.4 /  53.2    56.8 /  56.4     61.0 /  62.0
+//   FP32 N = 4   122 /   122 (15)  109 / 118 (10)  112 / 113 (0)
+// The packed and structure-of-arrays layouts (ADJ) have the same order, but FP32
+// UPWIND at N = 4 takes 118.0 in twos and 118.6 one by one.
+template <int N, class T, int FACES, bool ADJ> constexpr int face_chunk()
 {
-    return N <= 3 ? 5 : sizeof(T) == 8 ? 1 : 2;
+    if (N <= 3)
+        return 5;
+    return sizeof(T) == 8 || (FACES == FACES_UPWIND && !ADJ) ? 1 : 2;
 }
 template <int n, int CH, int F0, bool LF, int NFD, class T>
 __device__ __forceinline__ void face_fields(const FaceNodes<n, NFD, T> &fn, const FaceLine<n> &fl,
@@ -692,8 +704,11 @@ __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_wav
     // are first needed after P1: they are loaded with the neighbours' nodes
     // (prefetched, 37 VGPRs spilled).
     // With faces the tendencies stream past the L2, which the neighbours' reads
-    // need (N = 3 FP64 coastline 119 -> 115 us, N = 4 225 -> 216 us), except
-    // where a lane's nodes are adjacent and accesses share lines (246 -> 401).
+    // need, except where a lane's nodes are adjacent and accesses share lines
+    // (FP64 N = 3 246 -> 401 us).  Coastline octree, kept and streamed: FP64 N =
+    // 2 50.2 and 49.3, N = 3 101.2 and 96.4, N = 4 219.9 and 212.5 us; FP32 N = 3
+    // 55.5 and 53.4, N = 4 114.0 and 108.9 us; the same at N = 1, and FP32 N = 2
+    // 32.4 and 32.8 us.
     constexpr bool NTS = FACES != FACES_NONE && !ADJ;
     constexpr int NPRE = FACES && sizeof(TC) == 8 && N == 4 ? 3 : 5;
     // FP64 from N = 6 has no registers to load a step's initial state a phase
@@ -918,7 +933,7 @@ __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_wav
         }
         TC fa[FACES ? 5 : 1][n];
         if constexpr (FACES) {
-            constexpr int CH = face_chunk<N, TC>();
+            constexpr int CH = face_chunk<N, TC, FACES, ADJ>();
             FaceNodes<n, CH, TC> fn;
             fn.template load<0>(fl, U, L);
             __syncthreads();
