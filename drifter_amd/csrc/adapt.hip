@@ -30,8 +30,8 @@ __device__ __forceinline__ double wave_reduce_max(double v)
 
 // Lanes of a wavefront are split into groups of P = min(64, 2^ceil(log2 n^2))
 // lanes, one group per element; lane L of a group owns grid lines L, L + P, ...
-// (< n^2) of its element.  Element values are staged in the wave's LDS slice
-// with coalesced loads.
+// (< n^2) of its element.  A lane loads its xi-lines into registers and stages
+// them in the wave's LDS slice for the eta- and zeta-lines.
 struct LineMap {
     int P, epw, lpl; // group size, elements per wave, lines per lane
 };
@@ -93,7 +93,8 @@ __device__ __forceinline__ void wave_sync_lds()
 // Place of node (i, j, k) in an element's slice of LDS.  The LDS serves 16
 // doubles a clock; at n = 4 the 16 lines of an element, along any axis, met in
 // four banks each, so there the node's two low digits are crossed with k
-// (i ^ k and j ^ k are distinct over every line family).
+// (i ^ k and j ^ k are distinct over every line family).  Elsewhere the plain
+// place takes up to 2.5 clocks an access, but 8 for the xi-lines of n = 8.
 template <int n> __device__ __forceinline__ int place(int i, int j, int k)
 {
     if constexpr (n == 4)

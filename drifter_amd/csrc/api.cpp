@@ -183,7 +183,7 @@ drf_status volume(drf_ctx *c, const void *U, void *R, int layout, hipStream_t s,
 drf_status rhs_into(drf_ctx *c, const void *U, void *R, int layout, hipStream_t s)
 {
     // An attached face plan's conforming interfaces go into the volume
-    // kernel's last phase where the plan allows it; its mortars follow.
+    // kernel where the plan allows it; its mortars follow.
     VolFaces<double> f64{};
     VolFaces<float> f32{};
     const bool fused = c->faces && (c->precision == DRF_PREC_FP64

@@ -167,8 +167,8 @@ template <class T> struct Epi {
     double q[kMaxStages];
 };
 
-// The conforming face term fused into the volume kernel's last phase (a
-// face plan's element table; eface == nullptr: none).  Per element face:
+// The conforming face term inside the volume kernel, formed while a line is
+// in registers (a face plan's element table; eface == nullptr: none).  Per element face:
 // (neighbour << 1) | side, all ones where not conforming (side 0: this element
 // is the interface's left; a conforming neighbour always meets face f with its
 // opposite face f ^ 1).

@@ -45,7 +45,7 @@ struct drf_face_plan {
     std::vector<uint32_t> eface;
     int64_t *d_conf = nullptr, *d_mort = nullptr;
     uint32_t *d_eface = nullptr;
-    void *d_wq = nullptr;   // face-rule weight by face DOF (plan precision), for the fused phase
+    void *d_wq = nullptr;   // face-rule weight by face DOF (plan precision), for the volume kernel
     // conforming interfaces: DRF_FACES_BY_INTERFACE, _BY_ELEMENT or _IN_VOLUME
     int conf_mode = DRF_FACES_IN_VOLUME;
     void *d_ops[7] = {};       // per connection type: Minv | Pc | Lc | Pf[] | Lf[] (context precision)
