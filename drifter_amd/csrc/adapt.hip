@@ -135,7 +135,7 @@ template <int n> struct Lines1 {
 // directional mask; partial[block] = max of the block's values.  HBM-bound
 // (nd 8 + 17 B per element) once the LDS is out of the way: 196,400 elements,
 // N = 3 40.5 us with conflicting line reads and reductions through the LDS,
-// now 25.0 us.
+// now 24.6 us (fields that take turns; 22.4 us repeated on one).
 template <int n>
 __global__ void __launch_bounds__(64 * kWaves)
     estimate_kernel(int64_t E, const double *__restrict__ field, int64_t es,
