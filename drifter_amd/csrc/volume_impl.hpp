@@ -628,8 +628,9 @@ template <int n, int NFD, class T> struct FaceNodes {
 //   FP32 N = 2  32.8 /  32.4    33.0 /  33.6     35.4 /  35.8
 //   FP32 N = 3  53.4 /  53.2    56.8 /  56.4     61.0 /  62.0
 //   FP32 N = 4   122 /   122 (15)  109 / 118 (10)  112 / 113 (0)
-// The packed and structure-of-arrays layouts (ADJ) have the same order, but FP32
-// UPWIND at N = 4 takes 118.0 in twos and 118.6 one by one.
+// The packed and structure-of-arrays layouts (ADJ) agree, but for FP32: UPWIND at
+// N = 4 takes 118.0 in twos and 118.6 one by one, LF at N = 2 32.0 all at once and
+// 31.2 in twos (UPWIND 30.9 and 31.6).
 template <int N, class T, int FACES, bool ADJ> constexpr int face_chunk()
 {
     if (N <= 3)
@@ -725,8 +726,8 @@ __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_wav
     // The plain right-hand side's phases stand in a loop of one trip where the
     // compiler then keeps fewer bases and operators live across them (4 M nodes,
     // straight and in the loop: FP64 N = 6 133 and 113 us; FP32 N = 2 48.2 and
-    // 44.2, N = 3 42.4 and 41.0 us); it was slower at every other order (FP64
-    // N = 5 85 and 93, FP32 N = 4 46.5 and 50.3, N = 7 56 and 79 us).
+    // 44.2, N = 3 42.4 and 41.0 us); every other order was the same or slower
+    // (FP64 N = 5 85 and 93, FP32 N = 4 46.5 and 50.3, N = 7 56 and 79 us).
     constexpr bool ONE_TRIP = !STEP && FACES == FACES_NONE &&
                               (sizeof(TC) == 8 ? N == 6 : N == 2 || N == 3);
     constexpr int n2 = C::n2, n3 = C::n3, EPB = C::EPB;
@@ -1004,7 +1005,7 @@ __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_wav
         // ---------------- P3a: zeta-line (i, j) = L, momentum ----------------
         TC um[2][n]; // initial Hu, Hv for P4a
         if constexpr (step_reads_u0(EPI) && !LATE)
-            load_fields<n, 0, 2, ADJ, BY_FIELD>(U, state_off<EPB>(U, b, e, L), um);
+            load_fields<n, 0, 2, ADJ>(U, state_off<EPB>(U, b, e, L), um);
         {
             TC u[n], v[n], hi[n];
 #pragma unroll
@@ -1084,7 +1085,7 @@ __global__ void __launch_bounds__((Cfg<N, LW>::BLOCK)) __attribute__((amdgpu_wav
         // threads touch the same node of the same slot.
         TC ut[3][n]; // initial eta, HT, HS for P4b
         if constexpr (step_reads_u0(EPI) && !LATE)
-            load_fields<n, 2, 3, ADJ, BY_FIELD>(U, state_off<EPB>(U, b, e, L), ut);
+            load_fields<n, 2, 3, ADJ>(U, state_off<EPB>(U, b, e, L), ut);
         {
             TC ftv[n], fsv[n];
 #pragma unroll
